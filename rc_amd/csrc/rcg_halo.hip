@@ -142,15 +142,6 @@ __device__ __forceinline__ int run_key(int px)
   return (w - 1) + (h != w ? 32 : 0);
 }
 
-// The wavefront's next work item (-1 when all are drawn): the draw of
-// draw_item by lane 0, broadcast.
-__device__ __forceinline__ int next_item(int *q, int total, int &tried, int lane)
-{
-  int item = -1;
-  if (lane == 0) item = draw_item(q, total, blockIdx.x & 7, tried);
-  return __builtin_amdgcn_readfirstlane(item);
-}
-
 // Run table of a work item: lane `key` gets its key's first record (within
 // the item, whose records are sorted by key) and count.
 __device__ __forceinline__ void item_runs(const TiledDev &d, int item, int lane, int &first,
@@ -618,10 +609,10 @@ k_grid_halo(TiledDev d, const float2 *__restrict__ vis, const float2 *__restrict
   float2 *reg = sh.reg;
   const __amdgpu_buffer_rsrc_t rsrc = tap_rsrc(taps, n_taps);
   const int lane = threadIdx.x;
-  const int total = d.totals[1];
-  int tried = 0;
-  for (int item = next_item(d.queue, total, tried, lane); item >= 0;
-       item = next_item(d.queue, total, tried, lane)) {
+  ItemQueue iq(d.queue + Q_GRID, d.totals[1]);
+  int item = iq.first();
+  if (item < 0) item = iq.next();
+  for (; item >= 0; item = iq.next()) {
     const ItemRange ir = item_of(d, item);
     for (int q = lane; q < G::NC; q += 64) reg[q] = make_float2(0.f, 0.f);
     int first, count;
@@ -737,10 +728,10 @@ k_degrid_halo(TiledDev d, const float2 *__restrict__ grid, const float2 *__restr
   const __amdgpu_buffer_rsrc_t rsrc = tap_rsrc(taps, n_taps);
   const int lane = threadIdx.x;
   Sums out{sh.sums, sh.codes, vis, d.partial, (int)d.npts, lane};
-  const int total = d.totals[1];
-  int tried = 0;
-  for (int item = next_item(d.queue + 8, total, tried, lane); item >= 0;
-       item = next_item(d.queue + 8, total, tried, lane)) {
+  ItemQueue iq(d.queue + Q_DEGRID, d.totals[1]);
+  int item = iq.first();
+  if (item < 0) item = iq.next();
+  for (; item >= 0; item = iq.next()) {
     const ItemRange ir = item_of(d, item);
     const int gsz = d.grid_size;
     const float2 *gi = grid + ir.goff;
@@ -774,7 +765,7 @@ k_sort_items(TiledDev d)
   const int total = d.totals[1];
   while (true) {
     int item = 0;
-    if (lane == 0) item = atomicAdd(&d.queue[16], 1);
+    if (lane == 0) item = atomicAdd(&d.queue[Q_SORT], 1);
     item = __builtin_amdgcn_readfirstlane(item);
     if (item >= total) break;
     const ItemRange ir = item_of(d, item);

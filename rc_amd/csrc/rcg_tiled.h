@@ -16,9 +16,14 @@ constexpr int MAX_PLAN_TILES = 1 << 20;
 // Error word bit: a pair did not fit the plan's pair buffer (a chunk
 // support above the plan's max_support).
 constexpr int ERR_CAPACITY = 2;
-// Work-queue counters: [0, 8) gridding, [8, 16) degridding, one per XCD;
-// [16] the halo item sort.
+// Work-queue counters, QUEUE_STRIDE ints apart: 0..7 gridding, 8..15
+// degridding, one per XCD; 16 the halo item sort.  Each has a page of its own:
+// atomics from all XCDs to one line take about 12 ns each in turn, so with the
+// eight counters of a launch in one line a draw waited for those of every
+// XCD.
 constexpr int N_QUEUE = 17;
+constexpr int QUEUE_STRIDE = 1024;
+constexpr int Q_GRID = 0, Q_DEGRID = 8 * QUEUE_STRIDE, Q_SORT = 16 * QUEUE_STRIDE;
 
 // Records per work item of a halo-layout plan (its kernels sort an item's
 // records in LDS).
@@ -48,6 +53,7 @@ struct TiledDev {
   int *tile_start;   // first pair of each tile
   int *tile_cursor;  // fill cursors
   int *item_start;   // first work item of each tile
+  int4 *items;       // work items: first pair, end, tile, 1 if the tile's only one
   int *totals;       // [0] pairs, [1] items
   int *seg;          // scan scratch: 2 ints per segment of 1024 tiles
   int *queue;        // N_QUEUE work counters
@@ -59,7 +65,7 @@ struct TiledDev {
   float2 *lo;        // compensated flush: rounding errors of the atomic adds
   float2 *ibuf;      // halo gridding: each work item's region, items below
   int ibuf_cap;      // ibuf_cap (later items flush with atomics)
-  int item_cap;      // halo: bound on the number of work items
+  int item_cap;      // bound on the number of work items
   uint16_t *runs;    // halo: per work item, its records per run key (64)
   float2 *vsort;     // halo gridding: the visibility of every record, in record order
 };

@@ -78,21 +78,32 @@ __device__ __forceinline__ int4 make_pair(int u0, int v0, const rcg_pg &r, int p
 
 // ---------------------------------------------------------------------------
 // small utility kernels
-__global__ void k_fill_i32(int *__restrict__ p, int v, long long n)
+// Clears n floats at p and, when q is given, the eight work counters at q.
+__global__ void k_fill_f32(float *__restrict__ p, long long n, int *__restrict__ q)
 {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  for (; i < n; i += (long long)gridDim.x * blockDim.x) p[i] = v;
-}
-
-__global__ void k_fill_f32(float *__restrict__ p, long long n)
-{
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q && i < 8) q[i * QUEUE_STRIDE] = 0;
   const long long n4 = n >> 2;
   float4 *p4 = reinterpret_cast<float4 *>(p);
   for (long long k = i; k < n4; k += (long long)gridDim.x * blockDim.x)
     p4[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   for (long long k = (n4 << 2) + i; k < n; k += (long long)gridDim.x * blockDim.x)
     p[k] = 0.f;
+}
+
+// What binning counts into: tiles, totals, taps, error word and the halo item
+// sort's counter, in one launch (four launches of 4 us each before).
+__global__ void k_bin_clear(TiledDev d, unsigned long long *__restrict__ taps,
+                            int *__restrict__ err)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int t = i; t < d.n_tiles; t += gridDim.x * blockDim.x) d.tile_count[t] = 0;
+  if (i < 4) d.totals[i] = 0;
+  if (i == 0) {
+    *taps = 0;
+    *err = 0;
+    d.queue[Q_SORT] = 0;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -310,19 +321,45 @@ k_scan_top(TiledDev d, int n_seg)
   }
 }
 
+// Work items of the calling wavefront's tiles (one tile t per lane with c
+// pairs from p0 and m items from i0): a tile of up to 4 items by its lane,
+// the items of a larger one by all lanes.  With the table an item's range
+// costs one load; the search of the tile starts it replaces was a chain of
+// log2(tiles) loads per item.
+__device__ __forceinline__ void write_items(const TiledDev &d, int t, int c, int m, int p0, int i0)
+{
+  auto put = [&](int tile, int cnt, int first, int i, int k) {
+    if (i + k < d.item_cap)
+      d.items[i + k] = make_int4(first + k * d.chunk, first + min(cnt, (k + 1) * d.chunk), tile,
+                                 cnt <= d.chunk);
+  };
+  if (m <= 4)
+    for (int k = 0; k < m; k++) put(t, c, p0, i0, k);
+  const int lane = threadIdx.x & 63;
+  for (unsigned long long many = __ballot(m > 4); many; many &= many - 1) {
+    const int src = __ffsll(many) - 1;
+    const int tile = __shfl(t, src), cnt = __shfl(c, src), n = __shfl(m, src);
+    const int first = __shfl(p0, src), i = __shfl(i0, src);
+    for (int k = lane; k < n; k += 64) put(tile, cnt, first, i, k);
+  }
+}
+
 __global__ void __launch_bounds__(SCAN_SEG)
 k_scan_apply(TiledDev d)
 {
   __shared__ int2 sh[16];
   const int t = blockIdx.x * SCAN_SEG + threadIdx.x;
   const int c = t < d.n_tiles ? d.tile_count[t] : 0;
+  const int m = (c + d.chunk - 1) / d.chunk;
   int2 tot;
-  const int2 e = block_scan(make_int2(c, (c + d.chunk - 1) / d.chunk), sh, &tot);
+  const int2 e = block_scan(make_int2(c, m), sh, &tot);
+  const int p0 = d.seg[2 * blockIdx.x] + e.x, i0 = d.seg[2 * blockIdx.x + 1] + e.y;
   if (t < d.n_tiles) {
-    d.tile_start[t] = d.seg[2 * blockIdx.x] + e.x;
-    d.item_start[t] = d.seg[2 * blockIdx.x + 1] + e.y;
+    d.tile_start[t] = p0;
+    d.item_start[t] = i0;
     d.tile_cursor[t] = 0;
   }
+  write_items(d, t, c, m, p0, i0);
 }
 
 // Fill: LDS counts per tile within the workgroup, one global atomic per
@@ -495,7 +532,7 @@ k_grid_tiles(TiledDev d, const float2 *__restrict__ vis,
   // (measured: gridder kernel 2.83 -> 2.80 ms on the 4096^2 w-projection
   // workload)
   const int base = wave * CP * 8, dummy = vmove((wave * CP + DUMMY) * 8);
-  for_each_item(d, d.queue, [&](const ItemRange &ir) {
+  for_each_item(d, d.queue + Q_GRID, [&](const ItemRange &ir) {
     for (int q = threadIdx.x; q < GW * CP; q += 64 * GW) acc[q] = make_float2(0.f, 0.f);
     __syncthreads();
     const int npw = ir.end - ir.begin > wave ? (ir.end - ir.begin - wave + GW - 1) / GW : 0;
@@ -690,7 +727,7 @@ k_grid_tiles_f64(TiledDev d, const double2 *__restrict__ vis,
   __shared__ double2 acc[CP];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for_each_item(d, d.queue, [&](const ItemRange &ir) {
+  for_each_item(d, d.queue + Q_GRID, [&](const ItemRange &ir) {
     for (int q = threadIdx.x; q < CP; q += 64 * F64_WAVES) acc[q] = make_double2(0.0, 0.0);
     __syncthreads();
     for (int k = ir.begin + wave; k < ir.end; k += F64_WAVES) {
@@ -764,7 +801,7 @@ k_degrid_tiles_f64(TiledDev d, const double2 *__restrict__ grid,
   __shared__ double2 tile[T * LS];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for_each_item(d, d.queue + 8, [&](const ItemRange &ir) {
+  for_each_item(d, d.queue + Q_DEGRID, [&](const ItemRange &ir) {
     const int gsz = d.grid_size;
     const double2 *gi = grid + ir.goff;
     for (int q = threadIdx.x; q < T * T; q += 64 * F64_WAVES) {
@@ -855,7 +892,7 @@ k_degrid_tiles(TiledDev d, const float2 *__restrict__ grid,
   const int npts = (int)d.npts;
   float2 *my_sums = sums[wave];
   int *my_codes = codes[wave];
-  for_each_item(d, d.queue + 8, [&](const ItemRange &ir) {
+  for_each_item(d, d.queue + Q_DEGRID, [&](const ItemRange &ir) {
     const int gsz = d.grid_size;
     const float2 *gi = grid + ir.goff;
     for (int q = threadIdx.x; q < T * T; q += 64 * DW) {
@@ -1280,9 +1317,12 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
   if (e == hipSuccess) e = dalloc(&d.tile_start, (size_t)d.n_tiles);
   if (e == hipSuccess) e = dalloc(&d.tile_cursor, (size_t)d.n_tiles);
   if (e == hipSuccess) e = dalloc(&d.item_start, (size_t)d.n_tiles);
+  // work items: records / chunk + tiles at most
+  d.item_cap = (int)std::min(d.pair_cap / chunk + d.n_tiles, (long long)INT_MAX);
+  if (e == hipSuccess) e = dalloc(&d.items, (size_t)d.item_cap);
   if (e == hipSuccess) e = dalloc(&d.totals, 4);
   if (e == hipSuccess) e = dalloc(&d.seg, (size_t)2 * n_seg);
-  if (e == hipSuccess) e = dalloc(&d.queue, (size_t)N_QUEUE);
+  if (e == hipSuccess) e = dalloc(&d.queue, (size_t)N_QUEUE * QUEUE_STRIDE);
   if (e == hipSuccess) e = dalloc(&pl->taps, 1);
   if (e == hipSuccess) e = dalloc(&pl->err, 1);
   if (e == hipSuccess) e = dalloc(&d.pairs, (size_t)d.pair_cap);
@@ -1292,14 +1332,13 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
     // their number (records / chunk + tiles), within a 2 GiB budget; items
     // past it flush with atomics
     const long long cells = halo_region_cells(tile, wmax);
-    const long long bound = d.pair_cap / chunk + d.n_tiles;
     const long long budget = (2LL << 30) / (cells * (long long)sizeof(float2));
-    d.item_cap = (int)std::min(bound, (long long)INT_MAX);
-    d.ibuf_cap = (int)std::min(bound, budget);
+    d.ibuf_cap = (int)std::min((long long)d.item_cap, budget);
     e = dalloc(&d.ibuf, (size_t)(d.ibuf_cap * cells));
     if (e == hipSuccess) e = dalloc(&d.runs, (size_t)d.item_cap * 64);
     if (e == hipSuccess) e = dalloc(&d.vsort, (size_t)d.pair_cap);
   }
+  if (e == hipSuccess) e = hipMemset(d.totals, 0, 4 * sizeof(int));  // no items before binning
   if (e == hipSuccess)
     e = hipMemcpy(pl->geoms_dev, geoms, sizeof(rcg_geom) * n_inst, hipMemcpyHostToDevice);
   if (e == hipSuccess)
@@ -1337,7 +1376,7 @@ extern "C" rcg_status rcg_tiled_plan_destroy(rcg_tiled_plan *pl)
   if (!pl) return RCG_OK;
   TiledDev &d = pl->dev;
   void *ptrs[] = {pl->geoms_dev, pl->offs, pl->pg, d.tile_count, d.tile_start,
-                  d.tile_cursor, d.item_start, d.totals, d.seg, d.queue, pl->taps, pl->err,
+                  d.tile_cursor, d.item_start, d.items, d.totals, d.seg, d.queue, pl->taps, pl->err,
                   d.pairs, d.partial, pl->lo, d.ibuf, d.runs, d.vsort};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -1364,12 +1403,8 @@ extern "C" rcg_status rcg_tiled_bin(rcg_tiled_plan *pl, const rcg_gcf *gcf, void
   if (s != RCG_OK) return s;
   hipStream_t st = (hipStream_t)stream;
   TiledDev &d = pl->dev;
-  hipLaunchKernelGGL(k_fill_i32, dim3(256), dim3(256), 0, st, d.tile_count, 0,
-                     (long long)d.n_tiles);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, d.totals, 0, 4LL);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st,
-                     reinterpret_cast<int *>(pl->taps), 0, 2LL);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, pl->err, 0, 1LL);
+  hipLaunchKernelGGL(k_bin_clear, dim3(std::min(256, ceil_div(d.n_tiles, 256))), dim3(256), 0, st,
+                     d, pl->taps, pl->err);
   RCG_HIP_TRY(hipGetLastError());
   if (pl->n == 0) return RCG_OK;
   s = launch_pregrid_batch(pl->geoms_dev, d.pt_off, d.n_inst, pl->n, gcf, pl->pg, pl->taps,
@@ -1381,12 +1416,8 @@ extern "C" rcg_status rcg_tiled_bin(rcg_tiled_plan *pl, const rcg_gcf *gcf, void
 rcg_status rcg::tiled_bin_records(rcg_tiled_plan *pl, hipStream_t st)
 {
   TiledDev &d = pl->dev;
-  hipLaunchKernelGGL(k_fill_i32, dim3(256), dim3(256), 0, st, d.tile_count, 0,
-                     (long long)d.n_tiles);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, d.totals, 0, 4LL);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st,
-                     reinterpret_cast<int *>(pl->taps), 0, 2LL);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, pl->err, 0, 1LL);
+  hipLaunchKernelGGL(k_bin_clear, dim3(std::min(256, ceil_div(d.n_tiles, 256))), dim3(256), 0, st,
+                     d, pl->taps, pl->err);
   RCG_HIP_TRY(hipGetLastError());
   if (pl->n == 0) return RCG_OK;
   return bin_passes(pl, st);
@@ -1410,8 +1441,6 @@ rcg_status bin_passes(rcg_tiled_plan *pl, hipStream_t st)
                      pl->pg, d, pl->err);
   RCG_HIP_TRY(hipGetLastError());
   if (d.layout == LAYOUT_HALO) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, d.queue + 16, 0, 1LL);
-    RCG_HIP_TRY(hipGetLastError());
     return halo_sort_items(d, st);
   }
   return RCG_OK;
@@ -1436,11 +1465,11 @@ rcg_status grid_tiled(rcg_tiled_plan *pl, const rcg_gcf *gcf, const rcg_c64 *vis
   d.adj = adjoint;
   d.lo = pl->compensated ? pl->lo : nullptr;
   hipLaunchKernelGGL(k_fill_f32, dim3(2048), dim3(256), 0, st,
-                     reinterpret_cast<float *>(grid), d.gstride * d.n_inst * 2);
+                     reinterpret_cast<float *>(grid), d.gstride * d.n_inst * 2,
+                     d.queue + Q_GRID);
   if (d.lo)
     hipLaunchKernelGGL(k_fill_f32, dim3(2048), dim3(256), 0, st,
-                       reinterpret_cast<float *>(d.lo), d.gstride * d.n_inst * 2);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, d.queue, 0, 8LL);
+                       reinterpret_cast<float *>(d.lo), d.gstride * d.n_inst * 2, nullptr);
   RCG_HIP_TRY(hipGetLastError());
   if (pl->n == 0) return RCG_OK;
   const float2 *v = reinterpret_cast<const float2 *>(vis);
@@ -1520,8 +1549,7 @@ extern "C" rcg_status rcg_degrid_tiled_f32(rcg_tiled_plan *pl, const rcg_gcf *gc
   hipStream_t st = (hipStream_t)stream;
   const TiledDev &d = pl->dev;
   hipLaunchKernelGGL(k_fill_f32, dim3(1024), dim3(256), 0, st,
-                     reinterpret_cast<float *>(vis), pl->n * 2);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, d.queue + 8, 0, 8LL);
+                     reinterpret_cast<float *>(vis), pl->n * 2, d.queue + Q_DEGRID);
   RCG_HIP_TRY(hipGetLastError());
   if (pl->n == 0) return RCG_OK;
   const float2 *g = reinterpret_cast<const float2 *>(grid);
@@ -1577,10 +1605,9 @@ rcg_status grid_f64(rcg_tiled_plan *pl, const double2 *v, const double2 *t, long
   }
   d.adj = 0;
   d.lo = nullptr;
-  if (!add)
-    hipLaunchKernelGGL(k_fill_f32, dim3(2048), dim3(256), 0, st, reinterpret_cast<float *>(g),
-                       d.gstride * d.n_inst * 4);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, d.queue, 0, 8LL);
+  hipLaunchKernelGGL(k_fill_f32, dim3(add ? 1 : 2048), dim3(256), 0, st,
+                     reinterpret_cast<float *>(g), add ? 0LL : d.gstride * d.n_inst * 4,
+                     d.queue + Q_GRID);
   RCG_HIP_TRY(hipGetLastError());
   if (pl->n == 0) return RCG_OK;
   hipEvent_t *ev = timing_slot(pl, 0);
@@ -1622,8 +1649,7 @@ rcg_status degrid_f64(rcg_tiled_plan *pl, const double2 *g, const double2 *t, lo
   }
   // zeroed output: points left out stay 0, split windows add into it
   hipLaunchKernelGGL(k_fill_f32, dim3(2048), dim3(256), 0, st, reinterpret_cast<float *>(v),
-                     d.npts * 4);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, d.queue + 8, 0, 8LL);
+                     d.npts * 4, d.queue + Q_DEGRID);
   RCG_HIP_TRY(hipGetLastError());
   if (pl->n == 0) return RCG_OK;
   hipEvent_t *ev = timing_slot(pl, 1);

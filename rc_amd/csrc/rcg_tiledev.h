@@ -11,39 +11,6 @@ namespace rcg {
 // ---------------------------------------------------------------------------
 // work items
 
-// The largest t with item_start[t] <= item.  Tiles after the owning tile
-// start past `item`, so this is the owner (empty tiles before it share
-// smaller indices).
-__device__ __forceinline__ int find_tile(const int *__restrict__ item_start, int n_tiles,
-                                         int item)
-{
-  int lo = 0, hi = n_tiles - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (item_start[mid] <= item) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
-// Next work item of a workgroup (called by one thread).  The `total` items
-// are cut into 8 contiguous ranges, one per XCD: workgroups are dispatched
-// round-robin over the XCDs, so workgroup b runs on XCD b mod 8 and draws
-// from range b mod 8 first, then from the others in turn (`tried` counts
-// the ranges found empty).  Returns -1 when every range is used up; each
-// counter only grows, so every workgroup ends after at most 8 failed draws.
-__device__ __forceinline__ int draw_item(int *__restrict__ q, int total, int home, int &tried)
-{
-  const int per = (total + 7) >> 3;
-  while (tried < 8) {
-    const int x = (home + tried) & 7;
-    const int k = atomicAdd(&q[x], 1);
-    if (k < per && x * per + k < total) return x * per + k;
-    tried++;
-  }
-  return -1;
-}
-
 struct ItemRange {
   int item;                // index of the work item
   int begin, end, single;  // pairs [begin, end); the tile has one item
@@ -53,37 +20,110 @@ struct ItemRange {
 
 __device__ __forceinline__ ItemRange item_of(const TiledDev &d, int item)
 {
-  const int t = find_tile(d.item_start, d.n_tiles, item);
-  const int k = item - d.item_start[t];
-  const int cnt = d.tile_count[t];
+  const int4 it = d.items[item];
+  const int t = it.z;
   const int inst = t / d.tpi, lt = t - inst * d.tpi;
   ItemRange ir;
   ir.item = item;
-  ir.begin = d.tile_start[t] + k * d.chunk;
-  ir.end = d.tile_start[t] + min(cnt, (k + 1) * d.chunk);
-  ir.single = cnt <= d.chunk;
+  ir.begin = it.x;
+  ir.end = it.y;
+  ir.single = it.w;
   ir.tu0 = (lt / d.ntx) * d.T;
   ir.tv0 = (lt % d.ntx) * d.T;
   ir.goff = (long long)inst * d.gstride;
   return ir;
 }
 
+// Work items are drawn by one wavefront of a workgroup (all its lanes call;
+// every lane gets the result).  The `total` items are cut into 8 contiguous
+// ranges, one per XCD: workgroups are dispatched round-robin over the XCDs,
+// so workgroup b runs on XCD b mod 8 and draws from range b mod 8 first, then
+// from the others in turn.  The gridDim / 8 workgroups of a range own its
+// first items without a draw; counter x counts the draws from the rest of
+// range x.
+struct ItemQueue {
+  int *q;
+  int total, per, home, nhome;
+  bool home_open;  // no draw from the home range has failed yet
+
+  __device__ __forceinline__ ItemQueue(int *counters, int items)
+      : q(counters), total(items), per((items + 7) >> 3), home(blockIdx.x & 7),
+        nhome(gridDim.x >> 3)
+  {
+    home_open = drawn(home) > 0;
+  }
+  // Items of range x past those its workgroups own.
+  __device__ __forceinline__ int drawn(int x) const { return min(per, total - x * per) - nhome; }
+  // The workgroup's own item, -1 when its range is shorter.
+  __device__ __forceinline__ int first() const
+  {
+    const int k = blockIdx.x >> 3;
+    return k < per && home * per + k < total ? home * per + k : -1;
+  }
+  // The next item of any range; -1 when all are used up.  The home range is
+  // drawn from until that fails; then the counters are read, eight lanes at
+  // once, before one is drawn from, so that a workgroup that finds no items
+  // left leaves without an atomic: when every workgroup ended with a failed
+  // draw per range, the same-address atomics of 1536 workgroups
+  // held a launch for at least 150 us (195 us for 2048), most of the time of
+  // a small plan's gridding.  The counters only grow, so a retry finds fewer
+  // ranges left and every workgroup ends.
+  __device__ __forceinline__ int next()
+  {
+    const int lane = threadIdx.x & 63;
+    if (home_open) {
+      int k = 0;
+      if (lane == 0) k = atomicAdd(&q[home * QUEUE_STRIDE], 1);
+      k = __builtin_amdgcn_readfirstlane(k);
+      if (k < drawn(home)) return home * per + nhome + k;
+      home_open = false;
+    }
+    const int x = (home + lane) & 7;  // lane l looks at the l-th range to try
+    const int left = drawn(x);
+    while (true) {
+      int c = 0;
+      if (lane < 8 && left > 0)
+        c = __hip_atomic_load(&q[x * QUEUE_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned long long open = __ballot(lane < 8 && c < left);
+      if (!open) return -1;
+      const int src = __ffsll(open) - 1;
+      int k = 0;
+      if (lane == src) k = atomicAdd(&q[x * QUEUE_STRIDE], 1);
+      k = __builtin_amdgcn_readlane(k, src);
+      const int xs = (home + src) & 7;
+      if (k < drawn(xs)) return xs * per + nhome + k;
+    }
+  }
+};
+
 // Work loop of a persistent workgroup: fn(item range) for every item it
-// draws.  The trailing barrier keeps the next draw (and the next item's
-// LDS writes) behind every wavefront's use of the current one.
+// draws.  The trailing barrier keeps the next item's LDS writes behind every
+// wavefront's use of the current one.  The next draw waits for the end of an
+// item's work: made before it, it hides a latency of 1-2 us, but each
+// workgroup then holds an item in reserve while others run out (4096^2
+// w-projection workload, items of 140 us: 5.55 against 5.25 ms a step).
 template <class F>
 __device__ __forceinline__ void for_each_item(const TiledDev &d, int *__restrict__ q, F fn)
 {
   __shared__ int s_item;
-  const int total = d.totals[1];
-  int tried = 0;
-  while (true) {
-    if (threadIdx.x == 0) s_item = draw_item(q, total, blockIdx.x & 7, tried);
+  ItemQueue iq(q, d.totals[1]);
+  int item = iq.first();
+  if (item < 0) {
+    if (threadIdx.x < 64) {
+      item = iq.next();
+      if (threadIdx.x == 0) s_item = item;
+    }
     __syncthreads();
-    const int item = s_item;
-    if (item < 0) break;
+    item = s_item;
+  }
+  while (item >= 0) {
     fn(item_of(d, item));
+    if (threadIdx.x < 64) {
+      item = iq.next();
+      if (threadIdx.x == 0) s_item = item;
+    }
     __syncthreads();
+    item = s_item;
   }
 }
 
