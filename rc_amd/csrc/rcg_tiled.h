@@ -35,6 +35,8 @@ constexpr int LAYOUT_HALO = 1;   // one record per sub-window, in its origin's t
 
 struct TiledDev {
   int layout;        // LAYOUT_PAIRS or LAYOUT_HALO
+  int windows;       // pairs: slot 0's records carry the support for rcg_windows.hip,
+                     // up to this one (0: not that kind of plan)
   int wmax, lw;      // halo: largest sub-window side (16 or 32) and its log2
   int gbins;         // binning counts and ranks with global atomics (tiles
                      // per instance above the LDS histogram)
@@ -54,7 +56,7 @@ struct TiledDev {
   int *tile_cursor;  // fill cursors
   int *item_start;   // first work item of each tile
   int4 *items;       // work items: first pair, end, tile, 1 if the tile's only one
-  int *totals;       // [0] pairs, [1] items
+  int *totals;       // [0] pairs, [1] items, [3] points above d.windows
   int *seg;          // scan scratch: 2 ints per segment of 1024 tiles
   int *queue;        // N_QUEUE work counters
   const int *pt_off;   // n_inst + 1: first point of each instance
@@ -101,6 +103,15 @@ rcg_status halo_degrid(const TiledDev &d, int blocks, const float2 *grid, const 
 // items' run tables (the last pass of binning a halo-layout plan).
 rcg_status halo_sort_items(const TiledDev &d, hipStream_t st);
 
+// FP32 degridding of whole windows (rcg_windows.hip): whether a plan's tile
+// and supports fit its LDS, its persistent workgroups for `waves` (2, 4 or 8)
+// wavefronts each, and its launch.
+bool windows_fit(int T, int max_support);
+hipError_t windows_blocks(int T, int max_support, int waves, int *blocks);
+rcg_status windows_degrid(const TiledDev &d, int max_support, int waves, int blocks,
+                          const rcg_pg *pg, const float2 *grid, const float2 *taps,
+                          long long n_taps, float2 *vis, hipStream_t st);
+
 // FP64 gridding over the plan's pairs, added to the grid's contents.
 rcg_status tiled_grid_f64_add(rcg_tiled_plan *pl, const double2 *taps, long long n_taps,
                               const double2 *vis, double2 *grid, hipStream_t st);
@@ -114,6 +125,7 @@ struct rcg_tiled_plan {
   int max_support = 0;
   int max_pairs_pt = 0;
   int grid_waves = 0;     // wavefronts (private tile copies) per gridding workgroup
+  bool windows = false;   // FP32 degridding takes whole windows (rcg_windows.hip)
   int degrid_waves = 4;   // wavefronts per degridding workgroup (sharing the staged tile)
   int grid_blocks = 0;    // persistent workgroups of the grid kernel
   int degrid_blocks = 0;  // ... of the degrid kernel

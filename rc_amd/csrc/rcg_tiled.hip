@@ -52,8 +52,12 @@ namespace rcg {
 //      h:      intersection height (1..64)
 //      nslabs: 64-lane slabs of `rows` rows that cover it, ceil(h / rows)
 //   w: point index
+// In a plan that degrids whole windows (d.windows) nothing reads the slot;
+// the record of a point's first tile has bit 31 of z set and the point's
+// support, below 128, in the slot's bits and (its bit 6) in bit 30 of z, so
+// that the degridder needs no other record of the point.
 __device__ __forceinline__ int4 make_pair(int u0, int v0, const rcg_pg &r, int point,
-                                          int tile_r, int tile_c, int T, int slot)
+                                          int tile_r, int tile_c, int T, int slot, int windows)
 {
   const int S = r.supp, stride = r.stride;
   const int tu0 = tile_r * T, tv0 = tile_c * T;
@@ -73,6 +77,13 @@ __device__ __forceinline__ int4 make_pair(int u0, int v0, const rcg_pg &r, int p
   p.y = r.tap0 + (ra - u0) * stride + (ca - v0);
   p.z = stride | (h << 16) | (nslabs << 23);
   p.w = point;
+  if (windows) {
+    p.x &= ~(63 << 24);
+    if (slot == 0 && S <= windows) {
+      p.x |= (S & 63) << 24;
+      p.z |= (int)(0x80000000u | ((unsigned)S & 64) << 24);
+    }
+  }
   return p;
 }
 
@@ -116,22 +127,6 @@ __global__ void k_bin_clear(TiledDev d, unsigned long long *__restrict__ taps,
 // instance * tpi + row * ntx + column.
 
 constexpr int BIN_THREADS = 1024;
-
-// u0 = cell / pitch without an integer division: (cell + 0.5) / pitch lies
-// at least 0.5 / pitch (>= 2^-16) from an integer, and the FP64 product
-// (cell < 2^31) is within 2^-21 of it.
-__device__ __forceinline__ void point_tiles(const rcg_pg &r, int pitch, double inv_pitch, int lt,
-                                            int *u0, int *v0, int *tu0,
-                                            int *tu1, int *tv0, int *tv1)
-{
-  *u0 = (int)(((double)r.cell + 0.5) * inv_pitch);
-  *v0 = r.cell - *u0 * pitch;
-  const int S = r.supp;
-  *tu0 = *u0 >> lt;
-  *tu1 = (*u0 + S - 1) >> lt;
-  *tv0 = *v0 >> lt;
-  *tv1 = (*v0 + S - 1) >> lt;
-}
 
 struct BinBlock {
   int inst, p0, p1;  // points [p0, p1) of instance inst
@@ -197,7 +192,7 @@ __device__ __forceinline__ int point_records(const rcg_pg &r, int i, const Tiled
     int j = 0;
     for (int a = tu0; a <= tu1; a++)
       for (int b = tv0; b <= tv1; b++, j++)
-        f(a * d.ntx + b, j, make_pair(u0, v0, r, i, a, b, d.T, j));
+        f(a * d.ntx + b, j, make_pair(u0, v0, r, i, a, b, d.T, j, d.windows));
     return np;
   }
   const int S = r.supp, n = (S + d.wmax - 1) >> d.lw;
@@ -245,6 +240,9 @@ k_bin_count(const rcg_pg *__restrict__ pg, TiledDev d, int *__restrict__ err)
       atomicAdd(d.gbins ? &tc[t] : &hist[t], 1);
     });
     if (nr < 0) atomicOr(err, ERR_CAPACITY);  // support above the plan's max_support
+    // (one above it whose window meets no more tiles than the plan allows is
+    // taken, and degridded apart)
+    if (nr > 0 && d.windows && r.supp > d.windows) atomicOr(&d.totals[3], 1);
   }
   if (d.gbins) return;
   __syncthreads();
@@ -449,6 +447,8 @@ constexpr int grid_waves()
 {
   return T == 32 ? 3 : 4;
 }
+// Default wavefronts per degridding workgroup of a plan that degrids whole windows.
+constexpr int WINDOW_WAVES = 8;
 // Wavefronts per gridding workgroup a plan may choose (rcg_tiled_set_grid_waves).
 constexpr int MAX_GRID_WAVES = 4;
 
@@ -1307,6 +1307,12 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
         break;
     }
   }
+  pl->windows = !halo && windows_fit(tile, max_support);
+  d.windows = pl->windows ? max_support : 0;
+  if (e == hipSuccess && pl->windows) {
+    pl->degrid_waves = WINDOW_WAVES;
+    e = windows_blocks(tile, max_support, pl->degrid_waves, &pl->degrid_blocks);
+  }
   if (e == hipSuccess && halo &&
       halo_blocks(tile, wmax, &pl->grid_blocks, &pl->degrid_blocks) != RCG_OK)
     e = hipErrorInvalidValue;
@@ -1326,7 +1332,7 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
   if (e == hipSuccess) e = dalloc(&pl->taps, 1);
   if (e == hipSuccess) e = dalloc(&pl->err, 1);
   if (e == hipSuccess) e = dalloc(&d.pairs, (size_t)d.pair_cap);
-  if (e == hipSuccess) e = dalloc(&d.partial, (size_t)d.pair_cap);
+  if (e == hipSuccess && !pl->windows) e = dalloc(&d.partial, (size_t)d.pair_cap);
   if (e == hipSuccess && halo) {
     // item buffers of the halo gridder: every work item up to the bound on
     // their number (records / chunk + tiles), within a 2 GiB budget; items
@@ -1562,6 +1568,10 @@ extern "C" rcg_status rcg_degrid_tiled_f32(rcg_tiled_plan *pl, const rcg_gcf *gc
   if (d.layout == LAYOUT_HALO) {
     s = halo_degrid(d, pl->degrid_blocks, g, t, nt, v, st);
     if (s != RCG_OK) return s;
+  } else if (pl->windows) {
+    s = windows_degrid(d, pl->max_support, pl->degrid_waves, pl->degrid_blocks, pl->pg, g, t, nt,
+                       v, st);
+    if (s != RCG_OK) return s;
   } else {
     switch (d.T) {
       case 16: launch_degrid_tiles<16>(pl->degrid_waves, pl->degrid_blocks, d, g, t, nt, v, st); break;
@@ -1574,6 +1584,7 @@ extern "C" rcg_status rcg_degrid_tiled_f32(rcg_tiled_plan *pl, const rcg_gcf *gc
     RCG_HIP_TRY(hipEventRecord(ev[1], st));
     pl->n_ev[1]++;
   }
+  if (pl->windows) return RCG_OK;  // every point is whole
   hipLaunchKernelGGL(k_degrid_reduce, dim3((unsigned)((pl->n + 255) / 256)), dim3(256), 0, st,
                      d, pl->pg, pl->n, v);
   RCG_HIP_TRY(hipGetLastError());
@@ -1711,14 +1722,16 @@ extern "C" rcg_status rcg_tiled_set_degrid_waves(rcg_tiled_plan *pl, int waves)
               "runs one wavefront per workgroup");
     return RCG_ERR_UNSUPPORTED;
   }
-  if (waves == 0) waves = 4;
+  if (waves == 0) waves = pl->windows ? WINDOW_WAVES : 4;
   if (waves != 2 && waves != 4 && waves != 8) {
-    set_error(RCG_ERR_ARG, "rcg_tiled_set_degrid_waves: waves %d not 2, 4 or 8 (0: 4)", waves);
+    set_error(RCG_ERR_ARG, "rcg_tiled_set_degrid_waves: waves %d not 2, 4 or 8 (0: the default)",
+              waves);
     return RCG_ERR_ARG;
   }
   const int T = pl->dev.T;
   int nb = 0;
-  hipError_t e = T == 16 ? tile_kernels<16>(0, waves, nullptr, &nb)
+  hipError_t e = pl->windows ? windows_blocks(T, pl->max_support, waves, &nb)
+               : T == 16 ? tile_kernels<16>(0, waves, nullptr, &nb)
                : T == 32 ? tile_kernels<32>(0, waves, nullptr, &nb)
                          : tile_kernels<64>(0, waves, nullptr, &nb);
   RCG_HIP_TRY(e);

@@ -9,6 +9,25 @@
 namespace rcg {
 
 // ---------------------------------------------------------------------------
+// tiles of a point
+
+// u0 = cell / pitch without an integer division: (cell + 0.5) / pitch lies
+// at least 0.5 / pitch (>= 2^-16) from an integer, and the FP64 product
+// (cell < 2^31) is within 2^-21 of it.
+__device__ __forceinline__ void point_tiles(const rcg_pg &r, int pitch, double inv_pitch, int lt,
+                                            int *u0, int *v0, int *tu0,
+                                            int *tu1, int *tv0, int *tv1)
+{
+  *u0 = (int)(((double)r.cell + 0.5) * inv_pitch);
+  *v0 = r.cell - *u0 * pitch;
+  const int S = r.supp;
+  *tu0 = *u0 >> lt;
+  *tu1 = (*u0 + S - 1) >> lt;
+  *tv0 = *v0 >> lt;
+  *tv1 = (*v0 + S - 1) >> lt;
+}
+
+// ---------------------------------------------------------------------------
 // work items
 
 struct ItemRange {
