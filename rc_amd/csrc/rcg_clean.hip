@@ -10,34 +10,50 @@
 // (The reference's own findPeak reads past the array and returns |x|, so its
 // results are not reproduced; see the oracle.)
 //
-// GPU structure: one launch per iteration.  Every block of pass k first
-// reduces the block maxima that pass k - 1 left (512 entries of (|value|,
-// index, signed value): each block finds the same peak), applies the
-// threshold (block 0 updates the model and the state), subtracts the
-// peak's shifted PSF over its rows and leaves its own maximum of the
-// result (wavefront reductions on (|value|, -index)) in the other of two
-// buffers.  The kernel boundary orders the passes, so no block waits for
-// another and no device-wide fence is needed.  Peak, PSF peak, a stop flag
-// and the iteration count live in device memory, so no host
-// synchronisation is needed between iterations.
+// GPU structure.  Subtracting a component changes every pixel, but the peak
+// moves among few: the image is cut into at most 4096 square tiles, and a
+// tile is brought up to date (the components since its last visit subtracted,
+// in their order, its maximum found) only when it can hold the peak.  For
+// every tile the maximum e at its last visit and a slack s are kept, s the
+// sum of |a| times the largest |psf| over the part of the PSF that covered the
+// tile, for the components since.  Its maximum now is at most e + s, and the
+// image's at least the largest e - s; the tiles with e + s not below that are
+// visited, and more while one not visited could still exceed the best found.
+// So each iteration finds the same peak as a pass over the whole image, and
+// every pixel sees the same subtractions in the same order: the results are
+// bit for bit those of the passes.
 //
-// Measured, 1000 FP32 iterations on a 2048^2 dirty image: 17.8 ms with
-// 1024-thread blocks whose threads issue all 8 of their pixels' loads
-// together and keep a running maximum (24.4 ms with 256 threads and 4 loads
-// in flight, 18.4 ms without the running maximum).  Not taken: one
-// cooperative launch for the whole cycle, the residual held in registers and
-// a grid barrier per iteration, 27.0 ms; the barrier across the 8 XCDs
-// costs more than a kernel boundary.
-#include <cfloat>
-
+//   k_clean_tiles   one workgroup per tile: all pending components subtracted,
+//                   the tile's maximum (also the PSF's, with none pending);
+//   k_clean_prep    the PSF's peak and its tile maxima over 2 x 2 tiles;
+//   k_clean_minor   one workgroup, up to CK iterations: 4 tiles per thread in
+//                   registers, candidates visited by quarters, a
+//                   wavefront each;
+// then k_clean_tiles again.  No host synchronisation.
+//
+// What bounds it: k_clean_minor the latency of an iteration on one CU (three
+// barriers, one round of loads per visit), k_clean_tiles the reads of the PSF
+// beyond the L2 (16 MB a component at 2048^2 FP32, 10 TB/s).  Measured, 1000
+// FP32 iterations on a 2048^2 dirty image: 10.1 ms against 16.9 ms for one
+// pass over the whole image per iteration (a launch each, every block reducing
+// the last pass's 512 block maxima first); two major cycles of 100 iterations
+// at 1024^2: 2.2 against 4.2 ms.  CK iterations between two rounds of
+// k_clean_tiles: a tile seldom visited has up to CK components to catch up on,
+// a round costs 10 us besides them; 12 and 24 are within 1% of 16, 32 takes
+// 10.4, 64 11.4, 128 15.3 ms.  A visit's pixels four to a lane, loaded
+// together: 13 us an iteration at CK = 128, against 18 us one to a lane.
 #include "rcg_internal.h"
 
 namespace rcg {
 namespace {
 
-constexpr int CB = 512;   // blocks of the partial-maximum pass
-constexpr int CT = 1024;  // threads per block (at most; FP64 passes use 512)
-constexpr int PB = 8;     // pixels of a thread whose loads are issued together (a batch)
+constexpr int CT = 1024;       // threads of the one-workgroup kernels
+constexpr int CTILES = 4096;   // tiles of an image at most
+constexpr int PER = CTILES / CT;
+constexpr int CK = 16;         // iterations (components) between two rounds of k_clean_tiles
+constexpr int CAND = 128;      // tiles visited at a time
+constexpr int NP = 4;          // parts of a tile, a wavefront each
+constexpr int MSIDE = 65;      // side of the table of PSF maxima at most
 
 struct CleanState {
   long long pos;    // residual peak (row*pitch + col)
@@ -48,178 +64,475 @@ struct CleanState {
   int iters;
 };
 
-struct Best {
-  double a;        // |value|
-  long long idx;   // row-major index row*siz + col
-  double v;        // the signed value
+// A tile's maximum: |value|, the signed value, its place in the tile (row-major).
+struct TileMax {
+  double a, v;
+  int p, pad;
 };
 
-// Block maxima of one pass (CB entries).
-struct Partials {
-  double a[CB];
-  long long idx[CB];
-  double v[CB];
+struct Comp {
+  double a;    // amplitude times gain, as the image's type holds it
+  int dr, dc;  // row and column of the PSF over pixel (0, 0)
 };
 
-__device__ __forceinline__ Best better(Best x, Best y)
-{
-  if (y.a > x.a || (y.a == x.a && y.idx < x.idx)) return y;
-  return x;
-}
+struct Scratch {
+  CleanState st;
+  int nc;                    // pending components
+  int prow, pcol;            // PSF peak
+  Comp comp[CK];
+  unsigned char applied[CTILES];  // of the pending, how many a tile has had
+  TileMax psf[CTILES], res[CTILES];
+  float m2[MSIDE * MSIDE];   // largest |psf| over tiles (i-1, i) x (j-1, j)
+};
 
-__device__ __forceinline__ Best wave_best(Best b)
+// Tile geometry: nb x nb tiles of 2^lb pixels a side.
+struct Tiling {
+  int siz, pitch, lb, nb;
+};
+
+Tiling tiling_of(int siz, int pitch)
 {
-  for (int off = 32; off > 0; off >>= 1) {
-    Best o;
-    o.a = __shfl_xor(b.a, off);
-    o.idx = __shfl_xor(b.idx, off);
-    o.v = __shfl_xor(b.v, off);
-    b = better(b, o);
+  Tiling t{siz, pitch, 5, 0};
+  while (true) {
+    t.nb = (int)(((long long)siz + (1LL << t.lb) - 1) >> t.lb);
+    if ((long long)t.nb * t.nb <= CTILES) return t;
+    t.lb++;
   }
-  return b;
 }
 
-__device__ __forceinline__ Best block_best(Best b, Best *sh)
-{
-  b = wave_best(b);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) sh[wave] = b;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < (int)(blockDim.x >> 6); w++) b = better(b, sh[w]);
-    sh[0] = b;
-  }
-  __syncthreads();
-  return sh[0];
-}
-
-// The maximum of a pass's block maxima (every thread gets it).
-__device__ __forceinline__ Best reduce_partials(const Partials *__restrict__ p, Best *sh)
-{
-  Best b{-1.0, 0x7fffffffffffffffLL, 0.0};
-  for (int k = threadIdx.x; k < CB; k += blockDim.x) b = better(b, Best{p->a[k], p->idx[k], p->v[k]});
-  return block_best(b, sh);
-}
-
-// The PSF peak from the PSF's block maxima (one block).
-__global__ void __launch_bounds__(CT)
-k_clean_psf_peak(CleanState *__restrict__ st, int siz, int pitch,
-                 const Partials *__restrict__ pin)
-{
-  __shared__ Best sh[CT / 64];
-  const Best b = reduce_partials(pin, sh);
-  if (threadIdx.x != 0) return;
-  st->ppos = (b.idx / siz) * pitch + b.idx % siz;
-  st->pval = b.v;
-  st->done = 0;
-  st->iters = 0;
-}
-
-// Pass `it` over the image.  it >= 1: reduce pass it - 1's block maxima
-// (pin) to the peak of iteration it - 1; stop below the threshold; else
-// block 0 adds gain * peak / psf peak to the model, and every block
-// subtracts that times the PSF shifted onto the peak.  find: leave this
-// block's maximum of the (updated) image in pout.  it = 0: find only.
-// The image may be the PSF itself (it = 0, no subtraction).
+// Larger |value| first, then the lower place (a NaN is never larger).
 template <class T>
-__global__ void __launch_bounds__(CT)
-k_clean_pass(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ model, int siz,
-             int pitch, CleanState *__restrict__ st, double gain, double threshold, int it,
-             int find, const Partials *__restrict__ pin, Partials *__restrict__ pout)
+__device__ __forceinline__ void take(T &a, T &v, long long &p, T a2, T v2, long long p2)
+{
+  if (a2 > a || (a2 == a && p2 < p)) {
+    a = a2;
+    v = v2;
+    p = p2;
+  }
+}
+
+// One DPP step of a maximum over lanes: x and the lane that `CTRL` names.
+template <int CTRL, class T>
+__device__ __forceinline__ T dpp_max(T x)
+{
+  if constexpr (sizeof(T) == 8) {
+    const long long w = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp((int)w, (int)w, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(w >> 32), (int)(w >> 32), CTRL, 0xf, 0xf, false);
+    return fmax(x, __longlong_as_double((long long)hi << 32 | (unsigned)lo));
+  } else {
+    const int w = __float_as_int(x);
+    return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(w, w, CTRL, 0xf, 0xf, false)));
+  }
+}
+__device__ __forceinline__ long long lane_word(long long w, int l)
+{
+  const unsigned lo = __builtin_amdgcn_readlane((int)w, l);
+  const int hi = __builtin_amdgcn_readlane((int)(w >> 32), l);
+  return (long long)hi << 32 | lo;
+}
+__device__ __forceinline__ double lane_value(double x, int l)
+{
+  return __longlong_as_double(lane_word(__double_as_longlong(x), l));
+}
+__device__ __forceinline__ float lane_value(float x, int l)
+{
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+// Maximum over the wavefront (row_shr 1, 2, 4, 8, row_bcast 15, 31: in the
+// last lane) or, ROW, over each row of 16 lanes that hold the same values.
+// (Shuffles of the value, its sign and its place through LDS took 4 us a
+// workgroup; a few hundred cycles like this.)
+template <bool ROW, class T>
+__device__ __forceinline__ T lanes_max(T x)
+{
+  x = dpp_max<0x111>(x);
+  x = dpp_max<0x112>(x);
+  x = dpp_max<0x114>(x);
+  x = dpp_max<0x118>(x);
+  if (ROW) return lane_value(x, 15);
+  x = dpp_max<0x142>(x);
+  x = dpp_max<0x143>(x);
+  return lane_value(x, 63);
+}
+// The largest a (>= 0) of the lanes in `among`, the lowest place p on ties,
+// and its v; a = -1 when there is none.
+template <bool ROW, class T>
+__device__ __forceinline__ void lanes_best(T &a, T &v, long long &p, unsigned long long among)
+{
+  const T m = lanes_max<ROW>(a);
+  unsigned long long eq = m >= 0 ? __ballot(a == m) & among : 0;
+  T bv = 0;
+  long long bp = 0x7fffffffffffffffLL;
+  for (; eq; eq &= eq - 1) {
+    const int l = __ffsll(eq) - 1;
+    const long long q = lane_word(p, l);
+    if (q < bp) {
+      bp = q;
+      bv = lane_value(v, l);
+    }
+  }
+  a = m;
+  v = bv;
+  p = bp;
+}
+
+// Quarter q (by rows) of a tile, by one wavefront: components [k0, nc)
+// subtracted from its pixels, the largest of them (every lane gets it).  A
+// component lies over all of the part, over some of it, or not over it at
+// all; lane l finds out for the l-th of 64.  Those over all of it are taken
+// PC at a time: their loads are issued together, each from a scalar base (the
+// component's) and a lane offset (the pixel's), so that a pixel and component
+// cost one load and two operations.  (With the range tests of every pixel and
+// component instead, a visit was bound by instruction issue on its one CU.)
+template <int PC, class T>
+__device__ __forceinline__ TileMax visit(T *__restrict__ img, const T *__restrict__ psf,
+                                         const Tiling &g, int tile, int q, const Comp *comp, int k0,
+                                         int nc)
 {
 #pragma clang fp contract(off)
-  // separate slots for the two block reductions, so that the second one's
-  // writes cannot meet a slow wavefront's read of the first one's result
-  __shared__ Best sh_peak[CT / 64], sh_out[CT / 64];
-  long long dr = 0, dc = 0;
-  T a = 0;
-  const bool subtract = it > 0;
-  if (subtract) {
-    if (st->done) return;
-    const Best pk = reduce_partials(pin, sh_peak);
-    const long long r = pk.idx / siz, c = pk.idx % siz;
-    const long long pos = r * pitch + c;
-    const double pval = st->pval;
-    if (fabs(pk.v) < threshold || pval == 0.0) {
-      if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->pos = pos;
-        st->val = pk.v;
-        st->done = 1;
-      }
-      return;
-    }
-    const double g = gain * pk.v / pval;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      st->pos = pos;
-      st->val = pk.v;
-      st->iters = it;
-      model[pos] += (T)g;
-    }
-    const long long pr = st->ppos / pitch, pc = st->ppos % pitch;
-    dr = pr - r;
-    dc = pc - c;
-    a = (T)g;
-  }
-  // A thread's pixels are rows blockIdx.x + k * gridDim.x, columns
-  // threadIdx.x + j * blockDim.x, taken PB at a time in (k, j) order.  Every
-  // load of a batch (image, and PSF where the shifted PSF covers the pixel)
-  // is issued before any is used, so a batch costs one memory latency: at
-  // 2048^2 a thread's 8 pixels are one batch.  The pixels of a batch are
-  // distinct and img and psf do not alias, so the stores may follow all the
-  // loads.  The thread's running maximum: its pixels come in increasing index
-  // order, so a strict > keeps the first index on ties, as better() does.
+  // four pixels of a row per lane, one load of the image's own alignment
+  typedef T Quad __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const int lane = threadIdx.x & 63;
+  const int B = 1 << g.lb, rows = B / NP;
+  const int tr = tile / g.nb, tc = tile - tr * g.nb;
+  const int r0 = tr * B + q * rows, c0 = tc * B;
+  // the part's last row and column in the image
+  const int r1 = min(r0 + rows, g.siz) - 1, c1 = min(c0 + B, g.siz) - 1;
+  const bool wide = c0 + B <= g.siz;
   T ba = -1, bv = 0;
-  int br = -1, bc = 0;
-  const int tx = threadIdx.x, bx = blockIdx.x, nb = gridDim.x, nt = blockDim.x;
-  const int nj = tx < siz ? (siz - 1 - tx) / nt + 1 : 0;
-  const int nk = bx < siz ? (siz - 1 - bx) / nb + 1 : 0;
-  const int ne = nj * nk;
-  int k = 0, j = 0;
-  for (int e0 = 0; e0 < ne; e0 += PB) {
-    T x[PB], p[PB];
-    int rr[PB], cc[PB];
-    bool sb[PB];
+  int bp = 0x7fffffff;
+  for (int i = 0; i < rows << g.lb && r0 < g.siz; i += 256) {
+    const int p0 = i + lane * 4;
+    const int r = r0 + (p0 >> g.lb), c = c0 + (p0 & (B - 1));
+    // a lane past the edge works on the part's last pixels and drops them
+    const long long row = (long long)min(r, r1) * g.pitch;
+    auto load = [&](const T *src) {
+      Quad x;
+      if (wide) {
+        x = *reinterpret_cast<const Quad *>(src + (row + c));
+      } else {
 #pragma unroll
-    for (int u = 0; u < PB; u++) {
-      const int r = bx + k * nb, c = tx + j * nt;
-      const bool ok = e0 + u < ne;
-      const long long sr = r + dr, sc = c + dc;
-      rr[u] = r;
-      cc[u] = c;
-      sb[u] = ok && subtract && sr >= 0 && sr < siz && sc >= 0 && sc < siz;
-      x[u] = ok ? img[(long long)r * pitch + c] : T(0);
-      p[u] = sb[u] ? psf[sr * pitch + sc] : T(0);
-      if (++j == nj) {
-        j = 0;
-        k++;
+        for (int u = 0; u < 4; u++) x[u] = src[row + min(c + u, c1)];
+      }
+      return x;
+    };
+    Quad x = load(img);
+    for (int k = k0; k < nc; k += 64) {
+      const Comp mine = comp[min(k + lane, nc - 1)];
+      const T ma = (T)mine.a;
+      const bool live = k + lane < nc;
+      const bool some = live && r1 + mine.dr >= 0 && r0 + mine.dr < g.siz && c1 + mine.dc >= 0 &&
+                        c0 + mine.dc < g.siz;
+      const bool all = some && r0 + mine.dr >= 0 && r1 + mine.dr < g.siz && c0 + mine.dc >= 0 &&
+                       c1 + mine.dc < g.siz;
+      unsigned long long todo = __ballot(some);
+      const unsigned long long whole = __ballot(all);
+      while (todo) {
+        int l[PC];
+        unsigned long long left = todo, these = 0;
+#pragma unroll
+        for (int j = 0; j < PC; j++) {
+          l[j] = left ? __ffsll(left) - 1 : -1;
+          if (left) these |= left & -left;
+          left &= left - 1;
+        }
+        if ((these & ~whole) == 0) {
+          Quad y[PC];
+#pragma unroll
+          for (int j = 0; j < PC; j++) {
+            const int m = l[j] < 0 ? l[0] : l[j];
+            y[j] = load(psf + ((long long)__builtin_amdgcn_readlane(mine.dr, m) * g.pitch +
+                               __builtin_amdgcn_readlane(mine.dc, m)));
+          }
+#pragma unroll
+          for (int j = 0; j < PC; j++) {
+            if (l[j] < 0) break;
+            const T a = lane_value(ma, l[j]);
+#pragma unroll
+            for (int u = 0; u < 4; u++) x[u] -= a * y[j][u];
+          }
+          todo = left;
+        } else {
+          // one component, pixel by pixel
+          const int dr = __builtin_amdgcn_readlane(mine.dr, l[0]);
+          const int dc = __builtin_amdgcn_readlane(mine.dc, l[0]);
+          const T a = lane_value(ma, l[0]);
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const int sr = r + dr, sc = c + u + dc;
+            if (r <= r1 && c + u <= c1 && sr >= 0 && sr < g.siz && sc >= 0 && sc < g.siz)
+              x[u] -= a * psf[(long long)sr * g.pitch + sc];
+          }
+          todo &= todo - 1;
+        }
       }
     }
+    if (r <= r1) {
+      if (k0 < nc) {
+        if (wide) {
+          *reinterpret_cast<Quad *>(img + (row + c)) = x;
+        } else {
 #pragma unroll
-    for (int u = 0; u < PB; u++) {
-      if (sb[u]) {
-        x[u] -= a * p[u];
-        img[(long long)rr[u] * pitch + cc[u]] = x[u];
+          for (int u = 0; u < 4; u++)
+            if (c + u <= c1) img[row + c + u] = x[u];
+        }
       }
-      if (find && e0 + u < ne && fabs(x[u]) > ba) {
-        ba = fabs(x[u]);
-        bv = x[u];
-        br = rr[u];
-        bc = cc[u];
-      }
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        if (c + u <= c1 && fabs(x[u]) > ba) {
+          ba = fabs(x[u]);
+          bv = x[u];
+          bp = (q * rows << g.lb) + p0 + u;
+        }
     }
   }
-  if (!find) return;
-  Best b{-1.0, 0x7fffffffffffffffLL, 0.0};
-  if (br >= 0) b = Best{(double)ba, (long long)br * siz + bc, (double)bv};
-  // block maximum to thread 0 only (one barrier)
-  b = wave_best(b);
-  if ((tx & 63) == 0) sh_out[tx >> 6] = b;
+  long long p = bp;
+  lanes_best<false>(ba, bv, p, ~0ull);
+  return TileMax{(double)ba, (double)bv, ba >= 0 ? (int)p : 0x7fffffff, 0};
+}
+
+// One workgroup of 4 wavefronts per tile.  sc->nc pending components (which
+// == 0: the residual) or none (1: the PSF, read only).
+template <class T>
+__global__ void __launch_bounds__(256)
+k_clean_tiles(T *__restrict__ img, const T *__restrict__ psf, Tiling g, Scratch *__restrict__ sc,
+              int which, int pending)
+{
+  __shared__ Comp comp[CK];
+  __shared__ TileMax best[4];
+  const int nc = pending ? sc->nc : 0;
+  if (pending && nc == 0) return;  // stopped: nothing has changed
+  for (int k = threadIdx.x; k < nc; k += 256) comp[k] = sc->comp[k];
   __syncthreads();
-  if (tx == 0) {
-    for (int w = 1; w < (nt >> 6); w++) b = better(b, sh_out[w]);
-    pout->a[blockIdx.x] = b.a;
-    pout->idx[blockIdx.x] = b.idx;
-    pout->v[blockIdx.x] = b.v;
+  const int tile = blockIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int k0 = nc ? sc->applied[tile] : 0;
+  const TileMax m = visit<8>(img, psf, g, tile, wave, comp, k0, nc);
+  if ((threadIdx.x & 63) == 0) best[wave] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double a = best[0].a, v = best[0].v;
+    long long p = best[0].p;
+    for (int w = 1; w < 4; w++) take(a, v, p, best[w].a, best[w].v, (long long)best[w].p);
+    (which ? sc->psf : sc->res)[tile] = TileMax{a, v, (int)p, 0};
+  }
+}
+
+// The best of a workgroup's (a, v, p), in every thread.
+template <class T>
+struct BlockBest {
+  T a[CT / 64], v[CT / 64];
+  long long p[CT / 64];
+};
+template <class T>
+__device__ __forceinline__ void block_take(T &a, T &v, long long &p, BlockBest<T> &sh)
+{
+  lanes_best<false>(a, v, p, ~0ull);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) {
+    sh.a[wave] = a;
+    sh.v[wave] = v;
+    sh.p[wave] = p;
+  }
+  __syncthreads();
+  a = sh.a[lane & 15];
+  v = sh.v[lane & 15];
+  p = sh.p[lane & 15];
+  lanes_best<true>(a, v, p, 0xffffull);
+}
+
+constexpr long long NOWHERE = 0x7fffffffffffffffLL;
+
+// Row-major place in the image of place p of a tile.
+__device__ __forceinline__ long long image_place(const Tiling &g, int tile, int p)
+{
+  const int tr = tile / g.nb, tc = tile - tr * g.nb;
+  return (long long)((tr << g.lb) + (p >> g.lb)) * g.siz + (tc << g.lb) + (p & ((1 << g.lb) - 1));
+}
+
+// The PSF's peak and the table of its maxima; the state of a new cycle.
+__global__ void __launch_bounds__(CT)
+k_clean_prep(Tiling g, Scratch *__restrict__ sc)
+{
+  __shared__ BlockBest<double> sh;
+  const int nt = g.nb * g.nb;
+  double a = -1.0, v = 0.0;
+  long long p = NOWHERE;
+  for (int t = threadIdx.x; t < nt; t += CT) {
+    const TileMax m = sc->psf[t];
+    if (m.a >= 0.0) take(a, v, p, m.a, m.v, image_place(g, t, m.p));
+  }
+  block_take(a, v, p, sh);
+  if (threadIdx.x == 0) {
+    const bool any = p != NOWHERE;
+    const int pr = any ? (int)(p / g.siz) : 0, pc = any ? (int)(p % g.siz) : 0;
+    sc->st = CleanState{0, (long long)pr * g.pitch + pc, 0.0, any ? v : 0.0, 0, 0};
+    sc->prow = pr;
+    sc->pcol = pc;
+    sc->nc = 0;
+  }
+  const int side = g.nb + 1;
+  for (int k = threadIdx.x; k < side * side; k += CT) {
+    const int i = k / side, j = k - i * side;
+    float m = 0.f;
+    for (int di = -1; di <= 0; di++)
+      for (int dj = -1; dj <= 0; dj++) {
+        const int r = i + di, c = j + dj;
+        // rounded up
+        if (r >= 0 && r < g.nb && c >= 0 && c < g.nb)
+          m = fmaxf(m, (float)sc->psf[r * g.nb + c].a * 1.000001f);
+      }
+    sc->m2[k] = m;
+  }
+}
+
+// Up to `iters` (<= CK) iterations.  Three barriers an iteration: after the
+// candidates' list, the visits, and the new component.
+template <class T>
+__global__ void __launch_bounds__(CT)
+k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ model, Tiling g,
+              Scratch *__restrict__ sc, double gain, double threshold, int iters)
+{
+#pragma clang fp contract(off)
+  __shared__ float m2[MSIDE * MSIDE];
+  __shared__ Comp comp[CK];
+  __shared__ unsigned char applied[CTILES];
+  __shared__ int cand[CAND];
+  __shared__ TileMax found[CAND * NP];
+  __shared__ float sh_lb[CT / 64];
+  __shared__ int n_cand[2];  // the round's count; the other is cleared for the next
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (sc->st.done) {
+    if (tid == 0) sc->nc = 0;
+    return;
+  }
+  const int nt = g.nb * g.nb, side = g.nb + 1, prow = sc->prow, pcol = sc->pcol;
+  const double pval = sc->st.pval;
+  const int iter0 = sc->st.iters;
+  for (int k = tid; k < side * side; k += CT) m2[k] = sc->m2[k];
+  for (int t = tid; t < CTILES; t += CT) applied[t] = 0;
+  // Slacks in float, each step rounded up by more than the float operations
+  // and the rounding of the pixels' own subtractions can lose; above 0, so
+  // that a peak is always found by a visit.
+  constexpr float UP = 1.000001f, TINY = 5e-7f, LEAST = 1e-37f;
+  float e[PER], s[PER];
+  int at[PER], slot[PER];  // tile row << 16 | column (-1: no tile)
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const int t = tid + j * CT;
+    at[j] = t < nt ? (t / g.nb) << 16 | t % g.nb : -1;
+    e[j] = t < nt ? (float)sc->res[t].a * UP : -1.f;
+    s[j] = LEAST;
+  }
+  if (tid < 2) n_cand[tid] = 0;
+  int nc = 0, done = 0, flip = 0;
+  long long pos = 0;
+  double val = 0.0;
+  // A bound from below on the image's maximum: the largest e - s.
+  auto offer_lb = [&]() {
+    float lb = -1.f;
+#pragma unroll
+    for (int j = 0; j < PER; j++) lb = fmaxf(lb, e[j] * (1.f - 4.f * TINY) - s[j]);
+    lb = lanes_max<false>(lb);
+    if (lane == 0) sh_lb[wave] = lb;
+  };
+  offer_lb();
+  __syncthreads();
+  while (nc < iters) {
+    float lb = lanes_max<true>(sh_lb[lane & 15]);
+    T ba = -1, bv = 0;
+    long long bp = NOWHERE;
+    while (true) {
+      // tiles that can reach lb (a NaN slack: looked at)
+#pragma unroll
+      for (int j = 0; j < PER; j++) {
+        slot[j] = -1;
+        if (at[j] >= 0 && s[j] != 0.f && !(e[j] + s[j] < lb)) {
+          const int k = atomicAdd(&n_cand[flip], 1);
+          if (k < CAND) {
+            slot[j] = k;
+            cand[k] = tid + j * CT;
+          }
+        }
+      }
+      __syncthreads();
+      const int all = __builtin_amdgcn_readfirstlane(n_cand[flip]), n = min(all, CAND);
+      if (tid == 0) n_cand[flip ^ 1] = 0;
+      flip ^= 1;
+      for (int job = wave; job < n * NP; job += CT / 64) {
+        const int t = __builtin_amdgcn_readfirstlane(cand[job / NP]);
+        const TileMax m = visit<sizeof(T) == 4 ? 8 : 4>(
+            img, psf, g, t, job % NP, comp, __builtin_amdgcn_readfirstlane((int)applied[t]), nc);
+        if (lane == 0) found[job] = m;
+      }
+      __syncthreads();
+      // every wavefront: the best of the visits
+      for (int k = 0; k < n * NP; k += 64) {
+        T a = -1, v = 0;
+        long long p = NOWHERE;
+        if (k + lane < n * NP) {
+          const TileMax m = found[k + lane];
+          if (m.a >= 0.0) {
+            a = (T)m.a;
+            v = (T)m.v;
+            p = image_place(g, cand[(k + lane) / NP], m.p);
+          }
+        }
+        lanes_best<false>(a, v, p, ~0ull);
+        take(ba, bv, bp, a, v, p);
+      }
+#pragma unroll
+      for (int j = 0; j < PER; j++)
+        if (slot[j] >= 0) {
+          const TileMax *f = found + slot[j] * NP;
+          e[j] = (float)fmax(fmax(f[0].a, f[1].a), fmax(f[2].a, f[3].a)) * UP;
+          s[j] = 0.f;
+          applied[tid + j * CT] = (unsigned char)nc;
+        }
+      // Tiles not visited lie below lb: unless the list was full, or the best
+      // below lb (NaNs took pixels away), nothing can exceed the best found.
+      if (all <= CAND && ba >= lb) break;
+      if (all == 0) break;
+      lb = (float)ba * (1.f - 4.f * TINY);
+      __syncthreads();  // the list and the visits have been read
+    }
+    if (bp == NOWHERE || fabs((double)bv) < threshold || pval == 0.0) {
+      done = 1;
+      pos = bp == NOWHERE ? 0 : bp / g.siz * g.pitch + bp % g.siz;
+      val = bv;
+      break;
+    }
+    const int r = (int)(bp / g.siz), c = (int)(bp - (long long)r * g.siz);
+    const double w = gain * (double)bv / pval;
+    pos = (long long)r * g.pitch + c;
+    val = bv;
+    if (tid == 0) {
+      comp[nc] = Comp{(double)(T)w, prow - r, pcol - c};
+      model[pos] += (T)w;
+    }
+    nc++;
+    const float aw = fabsf((float)w) * UP;
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+      if (at[j] >= 0) {
+        // the tile's first row and column in the PSF, and the PSF tiles there
+        const int i = ((((at[j] >> 16) << g.lb) + prow - r) >> g.lb) + 1;
+        const int k = ((((at[j] & 0xffff) << g.lb) + pcol - c) >> g.lb) + 1;
+        const float m = i >= 0 && i < side && k >= 0 && k < side ? m2[i * side + k] : 0.f;
+        s[j] = (s[j] + aw * m + TINY * e[j] + LEAST) * UP;
+      }
+    offer_lb();
+    __syncthreads();
+  }
+  for (int k = tid; k < nc; k += CT) sc->comp[k] = comp[k];
+  for (int t = tid; t < nt; t += CT) sc->applied[t] = applied[t];
+  if (tid == 0) {
+    sc->nc = nc;
+    sc->st.pos = pos;
+    sc->st.val = val;
+    sc->st.done = done;
+    sc->st.iters = iter0 + nc;
   }
 }
 
@@ -235,27 +548,21 @@ template <class T>
 rcg_status hogbom(T *model, T *res, const T *psf, int siz, int pitch, unsigned niters,
                   double gain, double threshold, void *scratch, hipStream_t st)
 {
-  CleanState *cs = static_cast<CleanState *>(scratch);
-  Partials *pp = reinterpret_cast<Partials *>(cs + 1);  // two buffers, passes alternate
-  const long long n = (long long)siz * pitch;
-  // FP64 passes need more registers per thread (82 against 57 VGPRs at PB = 8):
-  // 512 threads keep two blocks per CU resident
-  const int nt = sizeof(T) == 8 ? 512 : CT;
-  hipLaunchKernelGGL(k_zero<T>, dim3(1024), dim3(256), 0, st, model, n);
-  // PSF peak
-  hipLaunchKernelGGL(k_clean_pass<T>, dim3(CB), dim3(nt), 0, st, const_cast<T *>(psf), psf,
-                     model, siz, pitch, cs, gain, threshold, 0, 1, pp + 1, pp);
-  hipLaunchKernelGGL(k_clean_psf_peak, dim3(1), dim3(CT), 0, st, cs, siz, pitch, pp);
-  if (niters == 0) {
-    RCG_HIP_TRY(hipGetLastError());
-    return RCG_OK;
+  Scratch *sc = static_cast<Scratch *>(scratch);
+  const Tiling g = tiling_of(siz, pitch);
+  const int nt = g.nb * g.nb;
+  hipLaunchKernelGGL(k_zero<T>, dim3(1024), dim3(256), 0, st, model, (long long)siz * pitch);
+  hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, const_cast<T *>(psf), psf, g,
+                     sc, 1, 0);
+  hipLaunchKernelGGL(k_clean_prep, dim3(1), dim3(CT), 0, st, g, sc);
+  if (niters > 0)
+    hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, res, psf, g, sc, 0, 0);
+  for (unsigned done = 0; done < niters; done += CK) {
+    const int n = (int)(niters - done < (unsigned)CK ? niters - done : (unsigned)CK);
+    hipLaunchKernelGGL(k_clean_minor<T>, dim3(1), dim3(CT), 0, st, res, psf, model, g, sc, gain,
+                       threshold, n);
+    hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, res, psf, g, sc, 0, 1);
   }
-  // pass 0: the maxima of the residual; pass it (1..niters): peak it - 1,
-  // its subtraction and, but for the last pass, the next maxima
-  for (unsigned it = 0; it <= niters; it++)
-    hipLaunchKernelGGL(k_clean_pass<T>, dim3(CB), dim3(nt), 0, st, res, psf, model, siz, pitch,
-                       cs, gain, threshold, (int)it, it < niters ? 1 : 0, pp + ((it + 1) & 1),
-                       pp + (it & 1));
   RCG_HIP_TRY(hipGetLastError());
   return RCG_OK;
 }
@@ -267,7 +574,7 @@ using namespace rcg;
 
 extern "C" size_t rcg_hogbom_scratch_bytes(void)
 {
-  return sizeof(CleanState) + 2 * sizeof(Partials);
+  return sizeof(Scratch);
 }
 
 extern "C" rcg_status rcg_hogbom(void *model, void *res, const void *psf, int f64, int siz,
