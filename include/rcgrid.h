@@ -451,8 +451,9 @@ rcg_status rcg_fft_plan_destroy(rcg_fft_plan *plan);
 rcg_status rcg_shutdown(void);
 
 /* GCF generation on device memory (the reference's mkGCFLayer and
- * calcAccums, GCF.cpp:16-219).  A generator owns the (8 max_support)^2
- * FP64 arena with row pitch 8 max_support + src_pad and its rocFFT plan;
+ * calcAccums, GCF.cpp:16-219).  A generator of the FP64 arena with side 8
+ * max_support and row pitch 8 max_support + src_pad (held in memory only for
+ * pad_quirk, whose sums walk it);
  * rcg_gcf_gen_layer writes one plane's 64 layers [8][8][support][support]
  * to dst (complex128 if f64, else complex64).  rcg_calc_accums: device uvw,
  * sums (double) and npts (int) of n_planes entries, err_dev one device int
@@ -461,6 +462,12 @@ typedef struct rcg_gcf_gen rcg_gcf_gen;
 rcg_status rcg_gcf_gen_create(int max_support, int src_pad, rcg_gcf_gen **gen);
 rcg_status rcg_gcf_gen_layer(rcg_gcf_gen *gen, void *dst, int f64, int support,
                              double t2, double w, int pad_quirk, void *stream);
+/* rcg_gcf_gen_layer for n planes (host arrays): plane k's layers of
+ * supports[k] for phase w[k] start at element offsets[k] of dst. */
+rcg_status rcg_gcf_gen_layers(rcg_gcf_gen *gen, void *dst, int f64, int n,
+                              const int *supports, const long long *offsets,
+                              double t2, const double *w, int pad_quirk,
+                              void *stream);
 rcg_status rcg_gcf_gen_destroy(rcg_gcf_gen *gen);
 rcg_status rcg_calc_accums(const rcg_double3 *uvw, long long n, double wstep,
                            int n_planes, double *sums, int *npts, int *err_dev,

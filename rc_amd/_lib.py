@@ -156,6 +156,8 @@ SIGNATURES: dict[str, tuple] = {
     "rcg_gcf_gen_create": (C.c_int, [C.c_int, C.c_int, C.POINTER(vp)]),
     "rcg_gcf_gen_layer": (C.c_int, [vp, vp, C.c_int, C.c_int, C.c_double, C.c_double, C.c_int,
                                     vp]),
+    "rcg_gcf_gen_layers": (C.c_int, [vp, vp, C.c_int, C.c_int, vp, vp, C.c_double, vp, C.c_int,
+                                     vp]),
     "rcg_gcf_gen_destroy": (C.c_int, [vp]),
     "rcg_calc_accums": (C.c_int, [vp, C.c_longlong, C.c_double, C.c_int, vp, vp, vp, vp]),
 }

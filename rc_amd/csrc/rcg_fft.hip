@@ -65,6 +65,17 @@ void fft_release()
   g_fft_plans--;
 }
 
+}  // namespace
+
+// GCF generators count as users of the state also before they make a plan.
+void fft_hold(int n)
+{
+  std::lock_guard<std::mutex> lk(g_fft_mu);
+  g_fft_plans += n;
+}
+
+namespace {
+
 // real <-> scratch copies for the reference's in-place strides
 template <class R>
 __global__ void k_real_rows(R *__restrict__ dst, int dpitch, const R *__restrict__ src,

@@ -23,11 +23,16 @@
 // Haskell caller uses src_pad = 4).  The default here is the pad-correct
 // sum; `pad_quirk` selects the reference's walk.
 //
-// GPU structure: one kernel writes the screen and zeroes the rest of the
-// arena (FP64 phase and sincos, contraction off); rocFFT does the
-// transform (rcg_fft plan, FP64, the reference's shift convention); 64
-// workgroups reduce the sub-lattice sums; one kernel divides and scatters
-// the window into the [8][8][S][S] layout (FP64 or complex64 output).
+// GPU structure.  Only max_support^2 cells of the arena differ from zero and
+// only support^2 samples per sub-lattice are kept, so the transform is two
+// small matrix products, out = E X E^T with E[u][a] = exp(2 pi i (u - L/2)
+// (a - R) / L) (L = 8 max_support, R = max_support / 2, X the screen): FP64
+// matrix instructions on 16 x 16 blocks, one launch for all planes of a table
+// (k_gcf_layers).  The sum over a sub-lattice needs no samples: the sum over
+// its max_support^2 places of E's products is max_support^2 for the cell
+// a = b = R, where the screen is 1, and 0 for every other.  With pad_quirk the
+// sums need the whole padded arena: screen, rocFFT (rcg_fft plan, made on
+// first use), 64 workgroups for the sums, one kernel for the window.
 // calcAccums uses per-workgroup LDS histograms and one FP64 atomic per
 // touched plane per workgroup.
 #include <algorithm>
@@ -41,12 +46,17 @@ constexpr int ACC_MAX_PLANES = 8192;
 
 struct rcg_gcf_gen {
   int max_support, src_pad, L, pitch;
+  bool held = false;         // counted as a user of the FFT library state
+  // pad_quirk only, made on first use
   double2 *arena = nullptr;  // L rows x pitch complex
   double *sums = nullptr;    // 64 sub-lattice sums
   rcg_fft_plan *fft = nullptr;
 };
 
 namespace rcg {
+// rcg_fft.hip: counts a user of the FFT library state (+1, -1).
+void fft_hold(int n);
+
 namespace {
 
 __global__ void __launch_bounds__(256)
@@ -74,11 +84,166 @@ k_wscreen(double2 *__restrict__ arena, int L, int pitch, int ms, double t2, doub
   }
 }
 
-// Sum of real parts over sub-lattice (over_u, over_v) = blockIdx.x: arena
-// cells (su*8 + over_u, sv*8 + over_v), su, sv < ms; with pad_quirk the
-// element at contiguous offset ((su*8 + over_u)*ms + sv)*8 + over_v.
+// One cell of the screen, (a, b) places from its centre.
+__device__ __forceinline__ double2 screen_cell(int a, int b, double normer, double w)
+{
+#pragma clang fp contract(off)
+  const double x = (double)a * normer, y = (double)b * normer;
+  const double ph = w * (1.0 - sqrt(1.0 - x * x - y * y));
+  double s, co;
+  sincos(2.0 * M_PI * ph, &s, &co);
+  return make_double2(co, -s);
+}
+
+// Planes of one launch.
+constexpr int GCF_PLANES = 64;
+struct GcfPlanes {
+  int n;
+  int support[GCF_PLANES];
+  int first[GCF_PLANES + 1];  // first workgroup of each plane
+  long long off[GCF_PLANES];  // element offset of its layers in dst
+  double w[GCF_PLANES];
+};
+
+constexpr int GCF_ROWS = 32;  // output rows of a workgroup
+
+// LDS of k_gcf_layers: E's L roots of unity, Y (GCF_ROWS x max_support,
+// padded to whole blocks; a row one more than a multiple of 16 cells, so that
+// the 16 rows of an operand start in different banks, except where that would
+// not fit) and, where it fits, the
+// screen's quadrant (the screen is even in both coordinates).
+__host__ __device__ inline int gcf_ypitch(int ms)
+{
+  return ((ms + 15) & ~15) + (ms > 240 ? 0 : 1);
+}
+size_t gcf_lds(int ms, bool quad)
+{
+  const size_t q = quad ? (size_t)(ms / 2 + 1) * (ms / 2 + 1) : 0;
+  return (8 * (size_t)ms + (size_t)GCF_ROWS * gcf_ypitch(ms) + q) * sizeof(double2);
+}
+constexpr size_t GCF_LDS = 160 * 1024;
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// acc += A B on 16 x 16 blocks, four complex products deep: A's row lane % 16,
+// B's column lane % 16, term lane / 16; the result's column lane % 16, rows
+// 4 i + lane / 16.
+__device__ __forceinline__ void mfma_c(d4 &re, d4 &im, double2 a, double2 b)
+{
+  re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, re, 0, 0, 0);
+  im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, im, 0, 0, 0);
+  re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, re, 0, 0, 0);
+  im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, im, 0, 0, 0);
+}
+
+// 32 rows u of one plane: Y = E X (each wavefront a share of the columns), then
+// Y E^T (each a share of the column blocks).  Output columns are taken in the
+// order (over_v, sv), so that 16 lanes write consecutive taps.  Bound by the
+// matrix units and, for small supports, by the screen and the roots, which
+// every workgroup computes (1089 + 512 sincos at max_support 64).  Measured
+// for planes -31..31 with supports 8..64 at max_support 64 (taps and sums):
+// GCF_FIGURES
+template <class T, bool QUAD>
 __global__ void __launch_bounds__(256)
-k_gcf_sums(const double2 *__restrict__ arena, int pitch, int ms, int pad_quirk,
+k_gcf_layers(GcfPlanes pl, int ms, double t2, T *__restrict__ out)
+{
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  double2 *root = reinterpret_cast<double2 *>(smem);
+  double2 *Y = root + 8 * ms;
+  const int yp = gcf_ypitch(ms), R = ms / 2, L = 8 * ms;
+  double2 *quad = Y + GCF_ROWS * yp;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, l4 = lane >> 4;
+  int p = 0;
+  while (p + 1 < pl.n && (int)blockIdx.x >= pl.first[p + 1]) p++;
+  const int S = pl.support[p];
+  const double w = pl.w[p], normer = t2 / (double)R;
+  T *dst = out + pl.off[p];
+  for (int k = threadIdx.x; k < L; k += 256) {
+    double s, c;
+    sincospi(2.0 * (double)k / (double)L, &s, &c);
+    root[k] = make_double2(c, s);
+  }
+  if (QUAD) {
+    const int qs = R + 1;
+    for (int k = threadIdx.x; k < qs * qs; k += 256)
+      quad[k] = screen_cell(k / qs, k % qs, normer, w);
+  }
+  __syncthreads();
+  auto screen = [&](int a, int b) {  // a, b in [0, ms), else 0
+    if (a >= ms || b >= ms) return make_double2(0.0, 0.0);
+    const int x = abs(a - R), y = abs(b - R);
+    return QUAD ? quad[x * (R + 1) + y] : screen_cell(x, y, normer, w);
+  };
+  auto mod = [&](int k) {  // into [0, L)
+    k %= L;
+    return k < 0 ? k + L : k;
+  };
+  const int n8 = 8 * S;                           // output rows and columns
+  const int start = (ms / 2 - S / 2) * GCF_OVER;  // of the window in the arena
+  const int row0 = ((int)blockIdx.x - pl.first[p]) * GCF_ROWS;
+  // this lane's two A rows of E: index of exp(2 pi i (u - L/2)(a - R) / L) at
+  // a = l4, and its step for a + 4
+  int e0[2], de[2];
+  for (int h = 0; h < 2; h++) {
+    const int u = mod(start + min(row0 + 16 * h + l16, n8 - 1) - L / 2);
+    e0[h] = mod(u * (l4 - R));
+    de[h] = mod(4 * u);
+  }
+  for (int b0 = wave * 16; b0 < ms; b0 += 64) {
+    d4 re[2] = {}, im[2] = {};
+    int e[2] = {e0[0], e0[1]};
+    for (int a = l4; a < ms + l4; a += 4) {
+      const double2 x = screen(a, b0 + l16);  // 0 past ms
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        mfma_c(re[h], im[h], root[e[h]], x);
+        e[h] += de[h];
+        e[h] -= e[h] >= L ? L : 0;
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        Y[(16 * h + 4 * i + l4) * yp + b0 + l16] = make_double2(re[h][i], im[h][i]);
+  }
+  __syncthreads();
+  const double sum = (double)ms * (double)ms;
+  for (int f0 = wave * 16; f0 < n8; f0 += 64) {
+    const int f = min(f0 + l16, n8 - 1);
+    const int ov = f / S, sv = f - ov * S;
+    const int v = mod(start + 8 * sv + ov - L / 2);
+    int e = mod(v * (l4 - R));
+    const int d = mod(4 * v);
+    d4 re[2] = {}, im[2] = {};
+    for (int b = l4; b < ms + l4; b += 4) {
+      const double2 x = b < ms ? root[e] : make_double2(0.0, 0.0);
+#pragma unroll
+      for (int h = 0; h < 2; h++) mfma_c(re[h], im[h], Y[(16 * h + l16) * yp + min(b, ms - 1)], x);
+      e += d;
+      e -= e >= L ? L : 0;
+    }
+    if (f0 + l16 >= n8) continue;
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int r = row0 + 16 * h + 4 * i + l4;
+        if (r >= n8) continue;
+        T o;
+        o.x = re[h][i] / sum;
+        o.y = im[h][i] / sum;
+        dst[((long long)((r & 7) * GCF_OVER + ov) * S + (r >> 3)) * S + sv] = o;
+      }
+  }
+}
+
+// Sum of real parts over sub-lattice (over_u, over_v) = blockIdx.x: the
+// elements at contiguous offset ((su*8 + over_u)*ms + sv)*8 + over_v, su, sv <
+// ms (the reference's walk, which takes the padded arena for a contiguous one).
+__global__ void __launch_bounds__(256)
+k_gcf_sums(const double2 *__restrict__ arena, int pitch, int ms,
            double *__restrict__ sums)
 {
   __shared__ double sh[4];
@@ -86,9 +251,7 @@ k_gcf_sums(const double2 *__restrict__ arena, int pitch, int ms, int pad_quirk,
   double acc = 0.0;
   for (int e = threadIdx.x; e < ms * ms; e += 256) {
     const int su = e / ms, sv = e - (e / ms) * ms;
-    const long long k = pad_quirk
-        ? ((long long)(su * GCF_OVER + ou) * ms + sv) * GCF_OVER + ov
-        : (long long)(su * GCF_OVER + ou) * pitch + sv * GCF_OVER + ov;
+    const long long k = ((long long)(su * GCF_OVER + ou) * ms + sv) * GCF_OVER + ov;
     acc += arena[k].x;
   }
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
@@ -177,6 +340,7 @@ extern "C" rcg_status rcg_gcf_gen_destroy(rcg_gcf_gen *g)
 {
   if (!g) return RCG_OK;
   if (g->fft) rcg_fft_plan_destroy(g->fft);
+  if (g->held) fft_hold(-1);
   if (g->arena) (void)hipFree(g->arena);
   if (g->sums) (void)hipFree(g->sums);
   delete g;
@@ -201,21 +365,110 @@ extern "C" rcg_status rcg_gcf_gen_create(int max_support, int src_pad, rcg_gcf_g
   g->src_pad = src_pad;
   g->L = max_support * GCF_OVER;
   g->pitch = g->L + src_pad;
+  fft_hold(1);
+  g->held = true;
+  *out = g;
+  return RCG_OK;
+}
+
+namespace {
+
+// The arena, sums and FFT plan of the pad_quirk path.
+rcg_status gen_arena(rcg_gcf_gen *g)
+{
+  if (g->fft) return RCG_OK;
   const size_t bytes = (size_t)g->L * g->pitch * sizeof(double2);
-  if (hipMalloc(reinterpret_cast<void **>(&g->arena), bytes) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&g->sums), 64 * sizeof(double)) != hipSuccess) {
-    g->arena = nullptr;
-    rcg_gcf_gen_destroy(g);
-    set_error(RCG_ERR_NOMEM, "rcg_gcf_gen_create: device arena of %zu bytes", bytes);
+  if ((!g->arena && hipMalloc(reinterpret_cast<void **>(&g->arena), bytes) != hipSuccess) ||
+      (!g->sums &&
+       hipMalloc(reinterpret_cast<void **>(&g->sums), 64 * sizeof(double)) != hipSuccess)) {
+    set_error(RCG_ERR_NOMEM, "rcg_gcf_gen: device arena of %zu bytes", bytes);
     return RCG_ERR_NOMEM;
   }
-  rcg_status s = rcg_fft_plan_create(1, 1, g->L, g->pitch, &g->fft);
-  if (s != RCG_OK) {
-    g->fft = nullptr;
-    rcg_gcf_gen_destroy(g);
-    return s;
+  return rcg_fft_plan_create(1, 1, g->L, g->pitch, &g->fft);
+}
+
+rcg_status quirk_layer(rcg_gcf_gen *g, void *dst, int f64, int support, double t2, double w,
+                       hipStream_t st)
+{
+  rcg_status s = gen_arena(g);
+  if (s != RCG_OK) return s;
+  const long long cells = (long long)g->L * g->pitch;
+  const int nb = (int)std::min<long long>((cells + 255) / 256, 2048);
+  hipLaunchKernelGGL(k_wscreen, dim3(nb), dim3(256), 0, st, g->arena, g->L, g->pitch,
+                     g->max_support, t2, w);
+  RCG_HIP_TRY(hipGetLastError());
+  s = rcg_fft_execute(g->fft, g->arena, st);
+  if (s != RCG_OK) return s;
+  hipLaunchKernelGGL(k_gcf_sums, dim3(64), dim3(256), 0, st, g->arena, g->pitch, g->max_support,
+                     g->sums);
+  const long long n = 64LL * support * support;
+  const int nb2 = (int)std::min<long long>((n + 255) / 256, 1024);
+  if (f64)
+    hipLaunchKernelGGL(k_gcf_extract<double2>, dim3(nb2), dim3(256), 0, st, g->arena, g->pitch,
+                       g->max_support, support, g->sums, static_cast<double2 *>(dst));
+  else
+    hipLaunchKernelGGL(k_gcf_extract<float2>, dim3(nb2), dim3(256), 0, st, g->arena, g->pitch,
+                       g->max_support, support, g->sums, static_cast<float2 *>(dst));
+  RCG_HIP_TRY(hipGetLastError());
+  return RCG_OK;
+}
+
+template <class T, bool QUAD>
+rcg_status launch_layers(const GcfPlanes &pl, int ms, double t2, void *dst, hipStream_t st)
+{
+  const size_t lds = gcf_lds(ms, QUAD);
+  RCG_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gcf_layers<T, QUAD>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)GCF_LDS));
+  hipLaunchKernelGGL((k_gcf_layers<T, QUAD>), dim3(pl.first[pl.n]), dim3(256), lds, st, pl, ms, t2,
+                     static_cast<T *>(dst));
+  RCG_HIP_TRY(hipGetLastError());
+  return RCG_OK;
+}
+
+}  // namespace
+
+extern "C" rcg_status rcg_gcf_gen_layers(rcg_gcf_gen *g, void *dst, int f64, int n,
+                                         const int *supports, const long long *offsets, double t2,
+                                         const double *w, int pad_quirk, void *stream)
+{
+  clear_error();
+  if (!g || !dst || n < 1 || !supports || !offsets || !w) {
+    set_error(RCG_ERR_ARG, "rcg_gcf_gen_layers: null argument or no plane");
+    return RCG_ERR_ARG;
   }
-  *out = g;
+  for (int k = 0; k < n; k++)
+    if (supports[k] < 1 || supports[k] > g->max_support || offsets[k] < 0) {
+      set_error(RCG_ERR_ARG, "plane %d: support %d outside [1, %d] or offset %lld", k, supports[k],
+                g->max_support, offsets[k]);
+      return RCG_ERR_ARG;
+    }
+  hipStream_t st = (hipStream_t)stream;
+  if (pad_quirk) {
+    for (int k = 0; k < n; k++) {
+      char *to = static_cast<char *>(dst) + offsets[k] * (f64 ? sizeof(double2) : sizeof(float2));
+      const rcg_status s = quirk_layer(g, to, f64, supports[k], t2, w[k], st);
+      if (s != RCG_OK) return s;
+    }
+    return RCG_OK;
+  }
+  const int ms = g->max_support;
+  const bool quad = gcf_lds(ms, true) <= GCF_LDS;
+  for (int k0 = 0; k0 < n; k0 += GCF_PLANES) {
+    GcfPlanes pl;
+    pl.n = std::min(GCF_PLANES, n - k0);
+    pl.first[0] = 0;
+    for (int k = 0; k < pl.n; k++) {
+      pl.support[k] = supports[k0 + k];
+      pl.off[k] = offsets[k0 + k];
+      pl.w[k] = w[k0 + k];
+      pl.first[k + 1] = pl.first[k] + (8 * pl.support[k] + GCF_ROWS - 1) / GCF_ROWS;
+    }
+    const rcg_status s = f64 ? (quad ? launch_layers<double2, true>(pl, ms, t2, dst, st)
+                                     : launch_layers<double2, false>(pl, ms, t2, dst, st))
+                             : (quad ? launch_layers<float2, true>(pl, ms, t2, dst, st)
+                                     : launch_layers<float2, false>(pl, ms, t2, dst, st));
+    if (s != RCG_OK) return s;
+  }
   return RCG_OK;
 }
 
@@ -228,28 +481,8 @@ extern "C" rcg_status rcg_gcf_gen_layer(rcg_gcf_gen *g, void *dst, int f64, int 
               g ? g->max_support : 0);
     return RCG_ERR_ARG;
   }
-  hipStream_t st = (hipStream_t)stream;
-  const long long cells = (long long)g->L * g->pitch;
-  const int nb = (int)std::min<long long>((cells + 255) / 256, 2048);
-  hipLaunchKernelGGL(k_wscreen, dim3(nb), dim3(256), 0, st, g->arena, g->L, g->pitch,
-                     g->max_support, t2, w);
-  RCG_HIP_TRY(hipGetLastError());
-  rcg_status s = rcg_fft_execute(g->fft, g->arena, stream);
-  if (s != RCG_OK) return s;
-  hipLaunchKernelGGL(k_gcf_sums, dim3(64), dim3(256), 0, st, g->arena, g->pitch,
-                     g->max_support, pad_quirk ? 1 : 0, g->sums);
-  const long long n = 64LL * support * support;
-  const int nb2 = (int)std::min<long long>((n + 255) / 256, 1024);
-  if (f64)
-    hipLaunchKernelGGL(k_gcf_extract<double2>, dim3(nb2), dim3(256), 0, st, g->arena,
-                       g->pitch, g->max_support, support, g->sums,
-                       static_cast<double2 *>(dst));
-  else
-    hipLaunchKernelGGL(k_gcf_extract<float2>, dim3(nb2), dim3(256), 0, st, g->arena,
-                       g->pitch, g->max_support, support, g->sums,
-                       static_cast<float2 *>(dst));
-  RCG_HIP_TRY(hipGetLastError());
-  return RCG_OK;
+  const long long off = 0;
+  return rcg_gcf_gen_layers(g, dst, f64, 1, &support, &off, t2, &w, pad_quirk, stream);
 }
 
 extern "C" rcg_status rcg_calc_accums(const rcg_double3 *uvw, long long n, double wstep,
