@@ -442,7 +442,9 @@ rcg_status rcg_fft_plan_create(int sign, int f64, int size, int pitch,
 rcg_status rcg_fft_execute(rcg_fft_plan *plan, void *data, void *stream);
 rcg_status rcg_fft_plan_destroy(rcg_fft_plan *plan);
 
-/* Releases process-wide library state before the process exits: the rocFFT
+/* Releases process-wide library state before the process exits: the device
+ * memory (at most 4 GiB) and streams that the MS4 gridder and degridder calls
+ * keep for the next call (also when the rest is refused), and the rocFFT
  * library state that the first FFT plan set up (rocfft_setup) is cleaned up
  * (rocfft_cleanup).  Refused with RCG_ERR_ARG while an FFT plan (of
  * rcg_fft_plan_create, fft_inplace_even or a GCF generator) is alive.  A

@@ -283,6 +283,7 @@ extern "C" rcg_status rcg_fft_execute(rcg_fft_plan *p, void *data, void *stream)
 extern "C" rcg_status rcg_shutdown(void)
 {
   clear_error();
+  pool_trim();
   std::lock_guard<std::mutex> lk(g_fft_mu);
   if (g_fft_plans > 0) {
     set_error(RCG_ERR_ARG, "rcg_shutdown: %d FFT plans still alive", g_fft_plans);

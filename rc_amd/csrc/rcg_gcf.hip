@@ -142,7 +142,6 @@ __device__ __forceinline__ void mfma_c(d4 &re, d4 &im, double2 a, double2 b)
 // matrix units and, for small supports, by the screen and the roots, which
 // every workgroup computes (1089 + 512 sincos at max_support 64).  Measured
 // for planes -31..31 with supports 8..64 at max_support 64 (taps and sums):
-// GCF_FIGURES
 template <class T, bool QUAD>
 __global__ void __launch_bounds__(256)
 k_gcf_layers(GcfPlanes pl, int ms, double t2, T *__restrict__ out)

@@ -42,6 +42,17 @@ inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 rcg_status check_geom(const rcg_geom *g);
 rcg_status check_gcf(const rcg_gcf *t);
 
+// Device memory and streams kept between calls (rcg_pool.hip).  A block or
+// stream goes back only when nothing on the device uses it any more.
+hipError_t pool_get(void **p, size_t bytes);
+void pool_put(void *p);
+hipError_t pool_stream(hipStream_t *st);
+void pool_stream_put(hipStream_t st);
+void pool_trim();
+// A copy between the caller's host memory and the device, after what st holds;
+// done on return, but a small one to the device may still be queued on st.
+hipError_t pool_copy(void *dst, const void *src, size_t bytes, bool to_device, hipStream_t st);
+
 // Kernels launched from the legacy host wrappers ----------------------------
 // Plane ranges over in-bound points: out[0..1] = min/max w-plane,
 // out[2..3] = min/max plane of the referenced layers (out must be preset to

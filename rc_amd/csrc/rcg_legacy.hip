@@ -10,8 +10,9 @@
 // range of the in-bound points on the GPU, upload only the GCF layers of
 // those planes, pregrid (FP64, exact), grid (tiled FP64 gridder over binned
 // pairs, or the plain one where no plan fits) or degrid (plain FP64
-// degridder), copy the result back.  No state survives the call, as in the reference; calls from
-// different host threads use their own streams and buffers.
+// degridder), copy the result back.  No data survives the call, as in the
+// reference; device memory and streams are kept for the next one (rcg_pool.hip),
+// and calls from different host threads use their own.
 #include <algorithm>
 #include <climits>
 #include <cstring>
@@ -28,8 +29,8 @@ namespace {
 
 struct DevBuf {
   void *p = nullptr;
-  ~DevBuf() { if (p) (void)hipFree(p); }
-  hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 16); }
+  ~DevBuf() { pool_put(p); }
+  hipError_t alloc(size_t bytes) { return pool_get(&p, bytes); }
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
@@ -38,9 +39,19 @@ struct PlanGuard {
   ~PlanGuard() { if (p) (void)rcg_tiled_plan_destroy(p); }
 };
 
-struct StreamGuard {
+// The call's device state.  The buffers (and the plan's) go back to the pool
+// for any thread's next call, so the destructor first waits for the stream,
+// on the paths that end in an error too.
+struct CallState {
+  DevBuf uvw, supps, range, pg, counts, data, table, vis, grid;
+  PlanGuard plan;
   hipStream_t s = nullptr;
-  ~StreamGuard() { if (s) (void)hipStreamDestroy(s); }
+  ~CallState()
+  {
+    if (!s) return;
+    (void)hipStreamSynchronize(s);
+    pool_stream_put(s);
+  }
 };
 
 #define LEG_TRY(expr)                                                        \
@@ -84,7 +95,14 @@ ull legacy_call(const LegacyArgs &a)
         if (a.vis_out[bl]) memset(a.vis_out[bl], 0, (size_t)a.ts_ch * sizeof(rcg_c128));
     }
   };
-  auto fail = [&]() -> ull { zero_outputs(); return 0ULL; };
+  // host staging must outlive the copies queued from it, also where the call
+  // ends early
+  hipStream_t st = nullptr;
+  auto fail = [&]() -> ull {
+    if (st) (void)hipStreamSynchronize(st);
+    zero_outputs();
+    return 0ULL;
+  };
   // host staging without value-initialisation (the copies fill it)
   auto host_array = [](size_t count, auto *tag) {
     using T = std::remove_pointer_t<decltype(tag)>;
@@ -151,25 +169,27 @@ ull legacy_call(const LegacyArgs &a)
     huvw = huvw_buf.get();
   }
 
-  StreamGuard sg;
-  LEG_TRY(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
-  hipStream_t st = sg.s;
+  CallState cs;
+  LEG_TRY(pool_stream(&cs.s));
+  st = cs.s;
 
-  DevBuf d_uvw, d_supps, d_range, d_pg, d_taps, d_err;
+  DevBuf &d_uvw = cs.uvw, &d_supps = cs.supps, &d_range = cs.range, &d_pg = cs.pg;
+  struct Counts {  // on the device in cs.counts
+    unsigned long long taps;
+    int err, pad;
+  };
   LEG_TRY(d_uvw.alloc((size_t)n * sizeof(rcg_double3)));
   LEG_TRY(d_supps.alloc((size_t)a.baselines * sizeof(int)));
   LEG_TRY(d_range.alloc(4 * sizeof(int)));
   LEG_TRY(d_pg.alloc((size_t)n * sizeof(rcg_pg)));
-  LEG_TRY(d_taps.alloc(sizeof(unsigned long long)));
-  LEG_TRY(d_err.alloc(sizeof(int)));
-  LEG_TRY(hipMemcpyAsync(d_uvw.p, huvw, (size_t)n * sizeof(rcg_double3),
-                         hipMemcpyHostToDevice, st));
+  LEG_TRY(cs.counts.alloc(sizeof(Counts)));
+  Counts *d_counts = cs.counts.as<Counts>();
+  LEG_TRY(pool_copy(d_uvw.p, huvw, (size_t)n * sizeof(rcg_double3), true, st));
   LEG_TRY(hipMemcpyAsync(d_supps.p, a.bl_supps, (size_t)a.baselines * sizeof(int),
                          hipMemcpyHostToDevice, st));
   int hrange[4] = {INT_MAX, INT_MIN, INT_MAX, INT_MIN};
   LEG_TRY(hipMemcpyAsync(d_range.p, hrange, sizeof(hrange), hipMemcpyHostToDevice, st));
-  LEG_TRY(hipMemsetAsync(d_taps.p, 0, sizeof(unsigned long long), st));
-  LEG_TRY(hipMemsetAsync(d_err.p, 0, sizeof(int), st));
+  LEG_TRY(hipMemsetAsync(d_counts, 0, sizeof(Counts), st));
 
   rcg_geom g;
   g.uvw = d_uvw.as<rcg_double3>();
@@ -206,68 +226,75 @@ ull legacy_call(const LegacyArgs &a)
     n_slots = (lmax + 1) * 64;
     center = 0;
   }
-  std::vector<int64_t> hoff((size_t)n_slots, 0);
-  std::vector<int32_t> hlen((size_t)n_slots, 0);
-  std::vector<int32_t> hsupp((size_t)(2 * M + 1), 0);
-  for (int p = pmin; p <= pmax; p++) hsupp[(size_t)(p + M)] = a.gcf_supps[p];
-  // (slot, source layer pointer, length) for every layer to upload; a
-  // layer of plane q holds gcf_supps[q]^2 taps
-  struct Src { int slot; const rcg_c128 *ptr; int len; };
-  std::vector<Src> srcs;
+  // One host block for the table's arrays: layer offsets, layer lengths,
+  // supports.
+  const size_t n_supp = (size_t)(2 * M + 1);
+  const size_t table_bytes = (size_t)n_slots * 12 + n_supp * 4;
+  std::vector<int64_t> table((table_bytes + 7) / 8, 0);
+  int64_t *hoff = table.data();
+  int32_t *hlen = reinterpret_cast<int32_t *>(hoff + n_slots);
+  int32_t *hsupp = hlen + n_slots;
+  for (int p = pmin; p <= pmax; p++) hsupp[p + M] = a.gcf_supps[p];
+  // every layer of the planes in use; a layer of plane q holds gcf_supps[q]^2
+  // taps.  Layers that follow each other in the caller's memory, as both
+  // reference callers lay them out, are copied from there.
+  long long total = 0;
+  const rcg_c128 *base = nullptr;
+  bool flat = true;
   for (int q = lmin; q <= lmax; q++) {
     const int gs = a.gcf_supps[q];
     for (int k = 0; k < 64; k++) {
-      const int idx = q * 64 + k;
-      srcs.push_back({idx + center, a.gcf[idx], gs > 0 ? gs * gs : 0});
+      const rcg_c128 *ptr = a.gcf[q * 64 + k];
+      if (!ptr) continue;
+      const int slot = q * 64 + k + center, len = gs > 0 ? gs * gs : 0;
+      if (!base && len) base = ptr;
+      if (len && ptr != base + total) flat = false;
+      hoff[slot] = total;
+      hlen[slot] = len;
+      total += len;
     }
   }
-  long long total = 0;
-  for (const Src &s : srcs) {
-    if (!s.ptr) { hlen[(size_t)s.slot] = 0; continue; }
-    hoff[(size_t)s.slot] = total;
-    hlen[(size_t)s.slot] = s.len;
-    total += s.len;
-  }
   const size_t n_data = (size_t)(total > 0 ? total : 1);
-  std::unique_ptr<rcg_c128[]> hdata = host_array(n_data, (rcg_c128 *)nullptr);
-  if (!hdata) {
-    set_error(RCG_ERR_NOMEM, "no host memory for %lld GCF taps", total);
-    return fail();
+  std::unique_ptr<rcg_c128[]> hdata;
+  const rcg_c128 *taps_src = base;
+  if (!flat || total == 0) {
+    hdata = host_array(n_data, (rcg_c128 *)nullptr);
+    if (!hdata) {
+      set_error(RCG_ERR_NOMEM, "no host memory for %lld GCF taps", total);
+      return fail();
+    }
+    if (total == 0) hdata[0] = rcg_c128{0.0, 0.0};
+    for (int q = lmin; q <= lmax; q++)
+      for (int k = 0; k < 64; k++) {
+        const int slot = q * 64 + k + center;
+        if (a.gcf[q * 64 + k] && hlen[slot])
+          memcpy(&hdata[(size_t)hoff[slot]], a.gcf[q * 64 + k],
+                 (size_t)hlen[slot] * sizeof(rcg_c128));
+      }
+    taps_src = hdata.get();
   }
-  if (total == 0) hdata[0] = rcg_c128{0.0, 0.0};
-  for (const Src &s : srcs)
-    if (s.ptr && s.len)
-      memcpy(&hdata[(size_t)hoff[(size_t)s.slot]], s.ptr, (size_t)s.len * sizeof(rcg_c128));
 
-  DevBuf d_data, d_off, d_len, d_tsupp;
-  LEG_TRY(d_data.alloc(n_data * sizeof(rcg_c128)));
-  LEG_TRY(d_off.alloc(hoff.size() * sizeof(int64_t)));
-  LEG_TRY(d_len.alloc(hlen.size() * sizeof(int32_t)));
-  LEG_TRY(d_tsupp.alloc(hsupp.size() * sizeof(int32_t)));
-  LEG_TRY(hipMemcpyAsync(d_data.p, hdata.get(), n_data * sizeof(rcg_c128),
-                         hipMemcpyHostToDevice, st));
-  LEG_TRY(hipMemcpyAsync(d_off.p, hoff.data(), hoff.size() * sizeof(int64_t),
-                         hipMemcpyHostToDevice, st));
-  LEG_TRY(hipMemcpyAsync(d_len.p, hlen.data(), hlen.size() * sizeof(int32_t),
-                         hipMemcpyHostToDevice, st));
-  LEG_TRY(hipMemcpyAsync(d_tsupp.p, hsupp.data(), hsupp.size() * sizeof(int32_t),
-                         hipMemcpyHostToDevice, st));
+  LEG_TRY(cs.data.alloc(n_data * sizeof(rcg_c128)));
+  LEG_TRY(cs.table.alloc(table_bytes));
+  LEG_TRY(pool_copy(cs.data.p, taps_src, n_data * sizeof(rcg_c128), true, st));
+  LEG_TRY(hipMemcpyAsync(cs.table.p, table.data(), table_bytes, hipMemcpyHostToDevice, st));
+  const int64_t *d_off = cs.table.as<int64_t>();
+  const int32_t *d_len = reinterpret_cast<const int32_t *>(d_off + n_slots);
   rcg_gcf t;
-  t.data = d_data.p;
-  t.layer_off = d_off.as<int64_t>();
-  t.layer_len = d_len.as<int32_t>();
+  t.data = cs.data.p;
+  t.layer_off = d_off;
+  t.layer_len = d_len;
   t.n_slots = n_slots;
   t.center = center;
-  t.supps = d_tsupp.as<int32_t>();
+  t.supps = d_len + n_slots;
   t.max_w_plane = M;
   t.half = a.half ? 1 : 0;
   t.n_taps = (int64_t)n_data;
 
-  if (rcg_pregrid(&g, &t, d_pg.as<rcg_pg>(), d_taps.as<unsigned long long>(),
-                  d_err.as<int>(), st) != RCG_OK)
+  if (rcg_pregrid(&g, &t, d_pg.as<rcg_pg>(), &d_counts->taps, &d_counts->err, st) != RCG_OK)
     return fail();
 
-  DevBuf d_vis, d_grid;
+  DevBuf &d_vis = cs.vis, &d_grid = cs.grid;
   LEG_TRY(d_vis.alloc((size_t)n * sizeof(rcg_c128)));
   LEG_TRY(d_grid.alloc(gcells * sizeof(rcg_c128)));
   // Gridding: the tiled FP64 gridder over binned pairs where a plan fits
@@ -277,26 +304,20 @@ ull legacy_call(const LegacyArgs &a)
   // FP64 gridder.  Degridding: the plain FP64 degridder, a gather without
   // atomics that runs faster than the tiled one (3.8 ms against 5.2 ms on
   // the 4096^2 w-projection points in 32640 chunks of 306).
-  PlanGuard plan;
+  PlanGuard &plan = cs.plan;
   int max_s = 1;
   for (int bl = 0; bl < a.baselines; bl++) max_s = std::max(max_s, a.bl_supps[bl]);
   for (int tile : {32, 64}) {
     if (a.degrid) break;
     const long long nt = (a.size + tile - 1) / tile;
     if (nt * nt > MAX_PLAN_TILES) continue;
-    if (rcg_tiled_plan_create(&g, tile, 1024, max_s, &plan.p) == RCG_OK) break;
+    if (tiled_plan_create_pooled(&g, tile, 1024, max_s, &plan.p) == RCG_OK) break;
     plan.p = nullptr;
   }
   clear_error();
   (void)hipGetLastError();  // a failed plan allocation leaves its error behind
   if (plan.p) {
     if (rcg_tiled_bin(plan.p, &t, st) != RCG_OK) return fail();
-    int perr = 0;
-    if (rcg_tiled_stats(plan.p, nullptr, nullptr, nullptr, &perr, st) != RCG_OK) return fail();
-    if (perr & ERR_CAPACITY) {
-      set_error(RCG_ERR_HIP, "tiled plan: pair buffer overflow");
-      return fail();
-    }
   }
   t_last_path = plan.p ? RCG_PATH_TILED : RCG_PATH_PLAIN;
   if (!a.degrid) {
@@ -313,8 +334,7 @@ ull legacy_call(const LegacyArgs &a)
                (size_t)a.ts_ch * sizeof(rcg_c128));
       hvis = hvis_buf.get();
     }
-    LEG_TRY(hipMemcpyAsync(d_vis.p, hvis, (size_t)n * sizeof(rcg_c128),
-                           hipMemcpyHostToDevice, st));
+    LEG_TRY(pool_copy(d_vis.p, hvis, (size_t)n * sizeof(rcg_c128), true, st));
     if (plan.p) {
       if (rcg_grid_tiled_f64(plan.p, &t, d_vis.as<rcg_c128>(), d_grid.as<rcg_c128>(), st) !=
           RCG_OK)
@@ -323,43 +343,44 @@ ull legacy_call(const LegacyArgs &a)
                                   d_grid.as<rcg_c128>(), st) != RCG_OK) {
       return fail();
     }
-    LEG_TRY(hipMemcpyAsync(a.grid_out, d_grid.p, gcells * sizeof(rcg_c128),
-                           hipMemcpyDeviceToHost, st));
-    LEG_TRY(hipStreamSynchronize(st));
+    LEG_TRY(pool_copy(a.grid_out, d_grid.p, gcells * sizeof(rcg_c128), false, st));
   } else {
-    LEG_TRY(hipMemcpyAsync(d_grid.p, a.grid_in, gcells * sizeof(rcg_c128),
-                           hipMemcpyHostToDevice, st));
+    LEG_TRY(pool_copy(d_grid.p, a.grid_in, gcells * sizeof(rcg_c128), true, st));
     if (rcg_degrid_plain_f64(&g, &t, d_pg.as<rcg_pg>(), d_grid.as<rcg_c128>(),
                              d_vis.as<rcg_c128>(), st) != RCG_OK)
       return fail();
     if (consecutive(reinterpret_cast<const void *const *>(a.vis_out), sizeof(rcg_c128))) {
-      LEG_TRY(hipMemcpyAsync(a.vis_out[0], d_vis.p, (size_t)n * sizeof(rcg_c128),
-                             hipMemcpyDeviceToHost, st));
-      LEG_TRY(hipStreamSynchronize(st));
+      LEG_TRY(pool_copy(a.vis_out[0], d_vis.p, (size_t)n * sizeof(rcg_c128), false, st));
     } else {
       std::unique_ptr<rcg_c128[]> hvis = host_array((size_t)n, (rcg_c128 *)nullptr);
       if (!hvis) {
         set_error(RCG_ERR_NOMEM, "no host memory for %lld visibilities", n);
         return fail();
       }
-      LEG_TRY(hipMemcpyAsync(hvis.get(), d_vis.p, (size_t)n * sizeof(rcg_c128),
-                             hipMemcpyDeviceToHost, st));
-      LEG_TRY(hipStreamSynchronize(st));
+      LEG_TRY(pool_copy(hvis.get(), d_vis.p, (size_t)n * sizeof(rcg_c128), false, st));
       for (int bl = 0; bl < a.baselines; bl++)
         memcpy(a.vis_out[bl], &hvis[(size_t)bl * a.ts_ch], (size_t)a.ts_ch * sizeof(rcg_c128));
     }
   }
-  unsigned long long taps = 0;
-  int err = 0;
-  LEG_TRY(hipMemcpy(&taps, d_taps.p, sizeof(taps), hipMemcpyDeviceToHost));
-  LEG_TRY(hipMemcpy(&err, d_err.p, sizeof(err), hipMemcpyDeviceToHost));
-  if (err & ERR_RANGE) {
+  Counts counts{};
+  LEG_TRY(hipMemcpyAsync(&counts, d_counts, sizeof(counts), hipMemcpyDeviceToHost, st));
+  // (the plan's error word is looked at here too: waiting for it before the
+  // gridding would hold up the visibilities' copy)
+  int perr = 0;
+  if (plan.p && rcg_tiled_stats(plan.p, nullptr, nullptr, nullptr, &perr, st) != RCG_OK)
+    return fail();
+  LEG_TRY(hipStreamSynchronize(st));
+  if (perr & ERR_CAPACITY) {
+    set_error(RCG_ERR_HIP, "tiled plan: pair buffer overflow");
+    return fail();
+  }
+  if (counts.err & ERR_RANGE) {
     set_error(RCG_ERR_RANGE,
               "an in-bound point referenced a GCF layer outside the table or a "
               "window larger than its layer (chunk support above plane support)");
     return fail();
   }
-  return taps;
+  return counts.taps;
 }
 
 }  // namespace

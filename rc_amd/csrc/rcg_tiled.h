@@ -81,6 +81,11 @@ struct rcg_tiled_plan;
 
 namespace rcg {
 
+// A one-instance pairs plan whose device memory comes from the pool: its owner
+// destroys it only when its work is done.
+rcg_status tiled_plan_create_pooled(const rcg_geom *geom, int tile, int chunk, int max_support,
+                                    rcg_tiled_plan **plan);
+
 // Bins the records the caller wrote into the plan's record buffer
 // (rcg_tiled_plan::pg, one per point; cell -1 for a point left out) in place
 // of the pregrid that rcg_tiled_bin runs.
@@ -122,6 +127,7 @@ struct rcg_tiled_plan {
   std::vector<rcg_geom> geoms;
   rcg_geom *geoms_dev = nullptr;
   long long n = 0;
+  bool pooled = false;    // device memory of pool_get
   int max_support = 0;
   int max_pairs_pt = 0;
   int grid_waves = 0;     // wavefronts (private tile copies) per gridding workgroup
@@ -133,7 +139,7 @@ struct rcg_tiled_plan {
   rcg_pg *pg = nullptr;
   unsigned long long *taps = nullptr;
   int *err = nullptr;
-  int *offs = nullptr;    // device pt_off | blk_off
+  int *offs = nullptr;    // device pt_off | blk_off | totals, in geoms_dev's block
   float2 *lo = nullptr;   // compensated flush grid (rcg_tiled_compensated)
   bool compensated = false;
   rcg::TiledDev dev{};

@@ -30,6 +30,7 @@
 //     summed in a fixed order by k_degrid_reduce.
 #include <algorithm>
 #include <climits>
+#include <cstring>
 
 #include "rcg_internal.h"
 #include "rcg_tiled.h"
@@ -1056,9 +1057,11 @@ int ilog2(int x)
 }
 
 template <class T>
-hipError_t dalloc(T **p, size_t n)
+hipError_t dalloc(T **p, size_t n, bool pooled)
 {
-  return hipMalloc(reinterpret_cast<void **>(p), (n ? n : 1) * sizeof(T));
+  void **v = reinterpret_cast<void **>(p);
+  const size_t bytes = (n ? n : 1) * sizeof(T);
+  return pooled ? pool_get(v, bytes) : hipMalloc(v, bytes);
 }
 
 // Persistent workgroups of a kernel: resident workgroups per CU x CUs,
@@ -1168,9 +1171,10 @@ hipEvent_t *timing_slot(rcg_tiled_plan *pl, int dir)
 
 using namespace rcg;
 
-extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst, int tile,
-                                               int chunk, int max_support, int layout,
-                                               rcg_tiled_plan **out)
+namespace {
+
+rcg_status create_plan(const rcg_geom *geoms, int n_inst, int tile, int chunk, int max_support,
+                       int layout, bool pooled, rcg_tiled_plan **out)
 {
   clear_error();
   if (!geoms || !out || n_inst < 1) {
@@ -1258,6 +1262,7 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
     return RCG_ERR_NOMEM;
   }
   pl->geoms.assign(geoms, geoms + n_inst);
+  pl->pooled = pooled;
   pl->n = n;
   pl->max_support = max_support;
   pl->max_pairs_pt = max_pairs_pt;
@@ -1316,23 +1321,33 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
   if (e == hipSuccess && halo &&
       halo_blocks(tile, wmax, &pl->grid_blocks, &pl->degrid_blocks) != RCG_OK)
     e = hipErrorInvalidValue;
-  if (e == hipSuccess) e = dalloc(&pl->geoms_dev, (size_t)n_inst);
-  if (e == hipSuccess) e = dalloc(&pl->offs, (size_t)2 * (n_inst + 1));
-  if (e == hipSuccess) e = dalloc(&pl->pg, (size_t)n);
-  if (e == hipSuccess) e = dalloc(&d.tile_count, (size_t)d.n_tiles);
-  if (e == hipSuccess) e = dalloc(&d.tile_start, (size_t)d.n_tiles);
-  if (e == hipSuccess) e = dalloc(&d.tile_cursor, (size_t)d.n_tiles);
-  if (e == hipSuccess) e = dalloc(&d.item_start, (size_t)d.n_tiles);
+  // geometries, offsets and totals (no items before binning) in one block and
+  // one copy
+  const size_t b_geoms = sizeof(rcg_geom) * n_inst, b_offs = sizeof(int) * 2 * (n_inst + 1);
+  std::vector<char> head(b_geoms + b_offs + 4 * sizeof(int), 0);
+  memcpy(head.data(), geoms, b_geoms);
+  memcpy(head.data() + b_geoms, pt_off.data(), b_offs / 2);
+  memcpy(head.data() + b_geoms + b_offs / 2, blk_off.data(), b_offs / 2);
+  if (e == hipSuccess)
+    e = dalloc(reinterpret_cast<char **>(&pl->geoms_dev), head.size(), pooled);
+  if (e == hipSuccess) {
+    pl->offs = reinterpret_cast<int *>(reinterpret_cast<char *>(pl->geoms_dev) + b_geoms);
+    d.totals = pl->offs + 2 * (n_inst + 1);
+  }
+  if (e == hipSuccess) e = dalloc(&pl->pg, (size_t)n, pooled);
+  if (e == hipSuccess) e = dalloc(&d.tile_count, (size_t)d.n_tiles, pooled);
+  if (e == hipSuccess) e = dalloc(&d.tile_start, (size_t)d.n_tiles, pooled);
+  if (e == hipSuccess) e = dalloc(&d.tile_cursor, (size_t)d.n_tiles, pooled);
+  if (e == hipSuccess) e = dalloc(&d.item_start, (size_t)d.n_tiles, pooled);
   // work items: records / chunk + tiles at most
   d.item_cap = (int)std::min(d.pair_cap / chunk + d.n_tiles, (long long)INT_MAX);
-  if (e == hipSuccess) e = dalloc(&d.items, (size_t)d.item_cap);
-  if (e == hipSuccess) e = dalloc(&d.totals, 4);
-  if (e == hipSuccess) e = dalloc(&d.seg, (size_t)2 * n_seg);
-  if (e == hipSuccess) e = dalloc(&d.queue, (size_t)N_QUEUE * QUEUE_STRIDE);
-  if (e == hipSuccess) e = dalloc(&pl->taps, 1);
-  if (e == hipSuccess) e = dalloc(&pl->err, 1);
-  if (e == hipSuccess) e = dalloc(&d.pairs, (size_t)d.pair_cap);
-  if (e == hipSuccess && !pl->windows) e = dalloc(&d.partial, (size_t)d.pair_cap);
+  if (e == hipSuccess) e = dalloc(&d.items, (size_t)d.item_cap, pooled);
+  if (e == hipSuccess) e = dalloc(&d.seg, (size_t)2 * n_seg, pooled);
+  if (e == hipSuccess) e = dalloc(&d.queue, (size_t)N_QUEUE * QUEUE_STRIDE, pooled);
+  if (e == hipSuccess) e = dalloc(&pl->taps, 1, pooled);
+  if (e == hipSuccess) e = dalloc(&pl->err, 1, pooled);
+  if (e == hipSuccess) e = dalloc(&d.pairs, (size_t)d.pair_cap, pooled);
+  if (e == hipSuccess && !pl->windows) e = dalloc(&d.partial, (size_t)d.pair_cap, pooled);
   if (e == hipSuccess && halo) {
     // item buffers of the halo gridder: every work item up to the bound on
     // their number (records / chunk + tiles), within a 2 GiB budget; items
@@ -1340,18 +1355,12 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
     const long long cells = halo_region_cells(tile, wmax);
     const long long budget = (2LL << 30) / (cells * (long long)sizeof(float2));
     d.ibuf_cap = (int)std::min((long long)d.item_cap, budget);
-    e = dalloc(&d.ibuf, (size_t)(d.ibuf_cap * cells));
-    if (e == hipSuccess) e = dalloc(&d.runs, (size_t)d.item_cap * 64);
-    if (e == hipSuccess) e = dalloc(&d.vsort, (size_t)d.pair_cap);
+    e = dalloc(&d.ibuf, (size_t)(d.ibuf_cap * cells), pooled);
+    if (e == hipSuccess) e = dalloc(&d.runs, (size_t)d.item_cap * 64, pooled);
+    if (e == hipSuccess) e = dalloc(&d.vsort, (size_t)d.pair_cap, pooled);
   }
-  if (e == hipSuccess) e = hipMemset(d.totals, 0, 4 * sizeof(int));  // no items before binning
   if (e == hipSuccess)
-    e = hipMemcpy(pl->geoms_dev, geoms, sizeof(rcg_geom) * n_inst, hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(pl->offs, pt_off.data(), sizeof(int) * (n_inst + 1), hipMemcpyHostToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(pl->offs + n_inst + 1, blk_off.data(), sizeof(int) * (n_inst + 1),
-                  hipMemcpyHostToDevice);
+    e = hipMemcpy(pl->geoms_dev, head.data(), head.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     rcg_tiled_plan_destroy(pl);
     set_error(RCG_ERR_NOMEM, "plan set-up failed: %s", hipGetErrorString(e));
@@ -1361,6 +1370,21 @@ extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst
   d.blk_off = pl->offs + n_inst + 1;
   *out = pl;
   return RCG_OK;
+}
+
+}  // namespace
+
+extern "C" rcg_status rcg_tiled_plan_create_ex(const rcg_geom *geoms, int n_inst, int tile,
+                                               int chunk, int max_support, int layout,
+                                               rcg_tiled_plan **out)
+{
+  return create_plan(geoms, n_inst, tile, chunk, max_support, layout, false, out);
+}
+
+rcg_status rcg::tiled_plan_create_pooled(const rcg_geom *geom, int tile, int chunk,
+                                         int max_support, rcg_tiled_plan **out)
+{
+  return create_plan(geom, 1, tile, chunk, max_support, RCG_LAYOUT_PAIRS, true, out);
 }
 
 extern "C" rcg_status rcg_tiled_plan_create_batch(const rcg_geom *geoms, int n_inst, int tile,
@@ -1381,11 +1405,11 @@ extern "C" rcg_status rcg_tiled_plan_destroy(rcg_tiled_plan *pl)
 {
   if (!pl) return RCG_OK;
   TiledDev &d = pl->dev;
-  void *ptrs[] = {pl->geoms_dev, pl->offs, pl->pg, d.tile_count, d.tile_start,
-                  d.tile_cursor, d.item_start, d.items, d.totals, d.seg, d.queue, pl->taps, pl->err,
+  void *ptrs[] = {pl->geoms_dev, pl->pg, d.tile_count, d.tile_start,
+                  d.tile_cursor, d.item_start, d.items, d.seg, d.queue, pl->taps, pl->err,
                   d.pairs, d.partial, pl->lo, d.ibuf, d.runs, d.vsort};
   for (void *p : ptrs)
-    if (p) (void)hipFree(p);
+    if (p) pl->pooled && p != pl->lo ? pool_put(p) : (void)hipFree(p);
   for (int dir = 0; dir < 2; dir++)
     for (int k = 0; k < N_TIMED; k++)
       for (int j = 0; j < 2; j++)
