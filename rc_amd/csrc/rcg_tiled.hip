@@ -439,15 +439,15 @@ constexpr int GRP = 2;
 // rcg_tiled_set_grid_waves; the autotuner searches it).  Each holds a
 // private copy of the tile in LDS, so the copies' size sets how many
 // workgroups share a CU's 160 KB: at T = 32 three wavefronts (25 KB) let six
-// workgroups (18 wavefronts) in, against four of four (16).  The default
-// below is the plan's choice until it is set: on the 4096^2 w-projection
-// workload 2, 3 and 4 wavefronts are within 1-2% of each other at T = 32,
-// one 3-5% slower; at T = 64 three copies leave one workgroup per CU.
-template <int T>
-constexpr int grid_waves()
-{
-  return T == 32 ? 3 : 4;
-}
+// workgroups (18 wavefronts) in, four (33 KB) four (16).  The default is the
+// plan's choice until it is set: four fill the four SIMDs evenly and walk an
+// item in 3/4 of the time, which is what a plan of few items waits for, and
+// a large plan loses nothing (gridder, three -> four: 100,000 points of 8 x 8
+// on 512^2 55 -> 43 us, 100,000 of 2..16 on 600^2 92 -> 77, 500,000 of 8..24
+// on 1024^2 122 -> 114, 4096^2 w-projection workload, chunk 1024, 2.52 ->
+// 2.46 ms).  Six or nine in a workgroup load the SIMDs unevenly (3.4 and
+// 4.4 ms); at T = 64 four copies are the one workgroup that fits a CU.
+constexpr int GRID_WAVES = 4;
 // Default wavefronts per degridding workgroup of a plan that degrids whole windows.
 constexpr int WINDOW_WAVES = 8;
 // Wavefronts per gridding workgroup a plan may choose (rcg_tiled_set_grid_waves).
@@ -1349,17 +1349,17 @@ rcg_status create_plan(const rcg_geom *geoms, int n_inst, int tile, int chunk, i
   if (e == hipSuccess && !halo) {
     switch (tile) {
       case 16:
-        pl->grid_waves = grid_waves<16>();
+        pl->grid_waves = GRID_WAVES;
         e = tile_kernels<16>(pl->grid_waves, pl->degrid_waves, &pl->grid_blocks,
                              &pl->degrid_blocks);
         break;
       case 32:
-        pl->grid_waves = grid_waves<32>();
+        pl->grid_waves = GRID_WAVES;
         e = tile_kernels<32>(pl->grid_waves, pl->degrid_waves, &pl->grid_blocks,
                              &pl->degrid_blocks);
         break;
       default:
-        pl->grid_waves = grid_waves<64>();
+        pl->grid_waves = GRID_WAVES;
         e = tile_kernels<64>(pl->grid_waves, pl->degrid_waves, &pl->grid_blocks,
                              &pl->degrid_blocks);
         break;
@@ -1776,7 +1776,7 @@ extern "C" rcg_status rcg_tiled_set_grid_waves(rcg_tiled_plan *pl, int waves)
     return RCG_ERR_ARG;
   }
   const int T = pl->dev.T;
-  if (waves == 0) waves = T == 16 ? grid_waves<16>() : T == 32 ? grid_waves<32>() : grid_waves<64>();
+  if (waves == 0) waves = GRID_WAVES;
   int nb = 0;
   hipError_t e = T == 16 ? tile_kernels<16>(waves, 0, &nb, nullptr)
                : T == 32 ? tile_kernels<32>(waves, 0, &nb, nullptr)

@@ -108,10 +108,13 @@ __device__ __forceinline__ void win_load(Steps &s, Walk &w, int dummy, __amdgpu_
   w.k += U;
 }
 
-// P = sum gx tx, Q = sum gy ty, R = sum gx ty, V = sum gy tx
+// P = sum gx tx, Q = sum gy ty, R = sum gx ty, V = sum gy tx, a set for each of
+// a pair's columns: chains half as long, whose rounding errors grow less.
+struct Acc {
+  float P[2], Q[2], R[2], V[2];
+};
 template <bool ODD>
-__device__ __forceinline__ void win_add(const Steps &s, const char *reg, float &P, float &Q,
-                                        float &R, float &V)
+__device__ __forceinline__ void win_add(const Steps &s, const char *reg, Acc &acc)
 {
   float2 g[U], h[U];
 #pragma unroll
@@ -127,14 +130,14 @@ __device__ __forceinline__ void win_add(const Steps &s, const char *reg, float &
       b = make_float2(0.f, 0.f);
       c = make_float2(0.f, 0.f);
     }
-    P = fmaf(g[u].x, s.a[u].x, P);
-    Q = fmaf(g[u].y, s.a[u].y, Q);
-    R = fmaf(g[u].x, s.a[u].y, R);
-    V = fmaf(g[u].y, s.a[u].x, V);
-    P = fmaf(c.x, b.x, P);
-    Q = fmaf(c.y, b.y, Q);
-    R = fmaf(c.x, b.y, R);
-    V = fmaf(c.y, b.x, V);
+    acc.P[0] = fmaf(g[u].x, s.a[u].x, acc.P[0]);
+    acc.Q[0] = fmaf(g[u].y, s.a[u].y, acc.Q[0]);
+    acc.R[0] = fmaf(g[u].x, s.a[u].y, acc.R[0]);
+    acc.V[0] = fmaf(g[u].y, s.a[u].x, acc.V[0]);
+    acc.P[1] = fmaf(c.x, b.x, acc.P[1]);
+    acc.Q[1] = fmaf(c.y, b.y, acc.Q[1]);
+    acc.R[1] = fmaf(c.x, b.y, acc.R[1]);
+    acc.V[1] = fmaf(c.y, b.x, acc.V[1]);
   }
 }
 
@@ -214,7 +217,7 @@ __device__ __forceinline__ void win_stream(const int4 *pts, int total, int wave,
   cb = nb;
   Steps s0, s1;
   load(s0);
-  float P = 0.f, Q = 0.f, R = 0.f, V = 0.f;
+  Acc acc = {};
   auto body = [&](Steps &cur, Steps &nxt) {
     if (lb == 0) {
       grp += W;
@@ -227,13 +230,14 @@ __device__ __forceinline__ void win_stream(const int4 *pts, int total, int wave,
     }
     load(nxt);
     __builtin_amdgcn_sched_barrier(0);
-    win_add<ODD>(cur, reg, P, Q, R, V);
+    win_add<ODD>(cur, reg, acc);
     if (--cb == 0) {
       // tap (tx, sg ty): re = P - sg Q, im = sg R + V
       const float sg = __int_as_float(0x3f800000 | ((conj << 1) & 0x80000000));
-      const float re = lane_sum(fmaf(-sg, Q, P)), im = lane_sum(fmaf(sg, R, V));
+      const float re = lane_sum(fmaf(-sg, acc.Q[0] + acc.Q[1], acc.P[0] + acc.P[1]));
+      const float im = lane_sum(fmaf(sg, acc.R[0] + acc.R[1], acc.V[0] + acc.V[1]));
       if (sub == G - 1 && point >= 0) vis[point] = make_float2(re, im);
-      P = Q = R = V = 0.f;
+      acc = {};
       point = npoint;
       conj = nconj;
       left--;

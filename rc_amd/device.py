@@ -181,7 +181,7 @@ class TiledPlan(_lib.Handle):
 
     def set_degrid_waves(self, waves: int) -> None:
         """Wavefronts per degridding workgroup, 2, 4 or 8; 0 restores the
-        default 4 (rcg_tiled_set_degrid_waves)."""
+        default (rcg_tiled_set_degrid_waves)."""
         _lib.check(_lib.lib().rcg_tiled_set_degrid_waves(self._h, int(waves)),
                    "rcg_tiled_set_degrid_waves")
         self.degrid_waves = int(waves)
