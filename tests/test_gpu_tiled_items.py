@@ -103,3 +103,24 @@ def test_window_degrid_above_max_support(hip_device):
     assert rel_l2(g.cpu().numpy(), ref) <= TOL
     assert rel_l2(v.cpu().numpy().reshape(70, 1), vref) <= TOL
     plan.close()
+
+
+@pytest.mark.parametrize("n,segments", [(512, 1), (528, 2), (2048, 16), (2064, 17), (2160, 18)])
+def test_scan_segments_vs_oracle(hip_device, n, segments):
+    """Windows over the whole of grids of 1, 2 and 16 segments of 1024 tiles
+    (one launch scans them) and of 17 and 18 (three launches), several items
+    per tile and a last segment that is not full."""
+    assert -(-(-(-n // 16)) ** 2 // 1024) == segments
+    vc, gcf, _ = synth.random_small(47, grid_size=n, chunks=500, ts_ch=4, half=True,
+                                    supports=(6, 8, 10), oob_frac=0.0)
+    rng = np.random.default_rng(n)
+    vc.uvw[..., :2] = rng.uniform(-n / 2 + 20, n / 2 - 20, vc.uvw[..., :2].shape) / vc.scale
+    vc, gcf = c64_round(vc, gcf)
+    ref, taps = O.grid(vc, gcf, n, nthreads=4)
+    gin = (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n)))
+    gin = gin.astype(np.complex64).astype(np.complex128)
+    vref, _ = O.degrid(vc, gcf, gin, nthreads=4)
+    g, v, st = run_tiled(vc, gcf, n, 16, 1, grid_in=gin)
+    assert st["err"] == 0 and st["taps"] == taps and st["items"] == st["pairs"] > 2000
+    assert rel_l2(g, ref) <= TOL
+    assert rel_l2(v, vref) <= TOL
