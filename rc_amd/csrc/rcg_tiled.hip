@@ -12,18 +12,21 @@
 //     edge appears in up to four tiles when S <= T).  A counting sort builds
 //     the per-tile lists without host synchronisation: LDS histograms per
 //     workgroup (each workgroup holds points of one instance) -> global
-//     counts -> three-kernel scan -> LDS-ranked fill;
+//     counts -> scan -> LDS-ranked fill;
 //  3. work items: each tile's list is cut into chunks of at most `chunk`
-//     pairs.  The grid and degrid kernels are persistent: a fixed number of
-//     workgroups draw items from eight queues, one per XCD, each holding a
-//     contiguous range of items (neighbouring tiles share that XCD's L2),
-//     and steal from the other queues when theirs is empty;
+//     pairs, a table holding every item's range.  The grid and degrid
+//     kernels are persistent: a fixed number of workgroups take items from
+//     eight ranges, one per XCD (neighbouring tiles share that XCD's L2),
+//     their first without a draw, then by a counter per range, their own
+//     range's first (ItemQueue);
 //  4. gridding: each wavefront accumulates its pairs' taps into a private
 //     FP32 copy of the tile in LDS, lanes covering the rows and columns of
 //     the window/tile intersection, GCF rows read coalesced; the copies
 //     are summed and stored to HBM with plain stores when the tile has a
 //     single item, with FP32 atomics (non-zero cells only) otherwise;
-//  5. degridding: the workgroup stages its grid tile in LDS, each wavefront
+//  5. degridding: by whole windows over a staged region of the grid where
+//     two workgroups' regions share a CU's LDS (rcg_windows.hip).  For larger
+//     supports the workgroup stages its grid tile in LDS, each wavefront
 //     forms per-lane partial sums of one pair over the intersection and
 //     reduces them across lanes four pairs at a time; points whose window
 //     lies in one tile are stored, split points leave one partial per tile,

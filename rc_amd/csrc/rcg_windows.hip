@@ -20,11 +20,11 @@
 // and loads wide.  A window cut at tile edges (k_degrid_tiles) fills 40 of 64
 // lanes with 8 bytes each, and leaves per-tile partial sums to store and add.
 // Measured on the 4096^2 w-projection workload (9,987,840 points, 3.2e9 taps):
-// 1.25 ms, 20 TB/s of taps, against 2.35 + 0.08 ms for k_degrid_tiles and its
-// sums; 16 snapshots of 2048^2 (6.3 M points): 0.79 against 1.65 ms.  Of the
-// 1.25 ms, 0.85 are the steps (1.15 of 1.35 without loads, so instruction
-// issue and the two workgroups per CU bound it), the rest the sorts and
-// staging of an item.  Variants on the former workload: 16 lanes a point 5%
+// 1.34 ms, 19 TB/s of taps, against 2.35 + 0.08 ms for k_degrid_tiles and its
+// sums; 16 snapshots of 2048^2 (6.3 M points): 0.89 against 1.65 ms.  With
+// FP32 sums (1.25 ms) 0.85 were the steps (1.15 of 1.35 without loads, so
+// instruction issue and the two workgroups per CU bound it), the rest the sorts
+// and staging of an item.  Variants on the former workload: 16 lanes a point 5%
 // slower, 32 lanes 24% (small windows leave them idle); U = 2 4% slower, 3
 // equal there and 5% slower on the latter; 4 wavefronts per workgroup 36%
 // slower; blocks that all lanes need without the range mask 5% slower; the
@@ -108,10 +108,14 @@ __device__ __forceinline__ void win_load(Steps &s, Walk &w, int dummy, __amdgpu_
   w.k += U;
 }
 
-// P = sum gx tx, Q = sum gy ty, R = sum gx ty, V = sum gy tx, a set for each of
-// a pair's columns: chains half as long, whose rounding errors grow less.
+// P = sum gx tx, Q = sum gy ty, R = sum gx ty, V = sum gy tx: the 2 U products
+// of a call in FP32, the calls' sums and the lanes' in FP64.  In FP32 a lane's
+// chain over the window would be S^2 / 8 long, eight times that of a wavefront
+// per window: relative L2 error of the 4096^2 workload's visibilities, six sets
+// of points, 0.67-2.9e-7 with FP32 sums per call, 0.68-2.2e-7 a wavefront per
+// window, 0.37-1.8e-7 this way, for 1.27 -> 1.34 ms.
 struct Acc {
-  float P[2], Q[2], R[2], V[2];
+  double P, Q, R, V;
 };
 template <bool ODD>
 __device__ __forceinline__ void win_add(const Steps &s, const char *reg, Acc &acc)
@@ -123,6 +127,7 @@ __device__ __forceinline__ void win_add(const Steps &s, const char *reg, Acc &ac
     g[u] = c[0];
     h[u] = c[1];
   }
+  float P = 0.f, Q = 0.f, R = 0.f, V = 0.f;
 #pragma unroll
   for (int u = 0; u < U; u++) {
     float2 b = s.b[u], c = h[u];
@@ -130,28 +135,34 @@ __device__ __forceinline__ void win_add(const Steps &s, const char *reg, Acc &ac
       b = make_float2(0.f, 0.f);
       c = make_float2(0.f, 0.f);
     }
-    acc.P[0] = fmaf(g[u].x, s.a[u].x, acc.P[0]);
-    acc.Q[0] = fmaf(g[u].y, s.a[u].y, acc.Q[0]);
-    acc.R[0] = fmaf(g[u].x, s.a[u].y, acc.R[0]);
-    acc.V[0] = fmaf(g[u].y, s.a[u].x, acc.V[0]);
-    acc.P[1] = fmaf(c.x, b.x, acc.P[1]);
-    acc.Q[1] = fmaf(c.y, b.y, acc.Q[1]);
-    acc.R[1] = fmaf(c.x, b.y, acc.R[1]);
-    acc.V[1] = fmaf(c.y, b.x, acc.V[1]);
+    P = u ? fmaf(g[u].x, s.a[u].x, P) : g[u].x * s.a[u].x;
+    Q = u ? fmaf(g[u].y, s.a[u].y, Q) : g[u].y * s.a[u].y;
+    R = u ? fmaf(g[u].x, s.a[u].y, R) : g[u].x * s.a[u].y;
+    V = u ? fmaf(g[u].y, s.a[u].x, V) : g[u].y * s.a[u].x;
+    P = fmaf(c.x, b.x, P);
+    Q = fmaf(c.y, b.y, Q);
+    R = fmaf(c.x, b.y, R);
+    V = fmaf(c.y, b.x, V);
   }
+  acc.P += P;
+  acc.Q += Q;
+  acc.R += R;
+  acc.V += V;
 }
 
 // Sum over a point's G lanes, in the last of them (fixed order).
-__device__ __forceinline__ float lane_sum(float x)
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double x)
 {
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, false));
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x112, 0xf, 0xf, false));
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x114, 0xf, 0xf, false));
-  if (G >= 16)
-    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x118, 0xf, 0xf, false));
-  if (G >= 32) x += __shfl_xor(x, 16);
-  if (G >= 64) x += __shfl_xor(x, 32);
-  return x;
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+  return x + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ float lane_sum(double x)
+{
+  static_assert(G == 8, "three steps");
+  return (float)dpp_add<0x114>(dpp_add<0x112>(dpp_add<0x111>(x)));
 }
 
 // A sorted point in LDS: x = tap offset of its window (elements), y = r0 |
@@ -233,9 +244,9 @@ __device__ __forceinline__ void win_stream(const int4 *pts, int total, int wave,
     win_add<ODD>(cur, reg, acc);
     if (--cb == 0) {
       // tap (tx, sg ty): re = P - sg Q, im = sg R + V
-      const float sg = __int_as_float(0x3f800000 | ((conj << 1) & 0x80000000));
-      const float re = lane_sum(fmaf(-sg, acc.Q[0] + acc.Q[1], acc.P[0] + acc.P[1]));
-      const float im = lane_sum(fmaf(sg, acc.R[0] + acc.R[1], acc.V[0] + acc.V[1]));
+      const double sg = (conj >> 30) & 1 ? -1.0 : 1.0;
+      const float re = lane_sum(fma(-sg, acc.Q, acc.P));
+      const float im = lane_sum(fma(sg, acc.R, acc.V));
       if (sub == G - 1 && point >= 0) vis[point] = make_float2(re, im);
       acc = {};
       point = npoint;
