@@ -737,10 +737,11 @@ k_grid_tiles(TiledDev d, const float2 *__restrict__ vis,
 // at T = 32 a copy is 17 KB, so nine workgroups fit a CU.  Real and imaginary
 // parts lie in planes of their own: 64 lanes on consecutive cells take 9
 // cycles an atomic there and 17 interleaved.  Records come 64 at a time and
-// the next pair's first taps fly while a pair is added.  Measured, 2,496,960
-// points of supports 8..48 in chunks of 306 on 2048^2 (330 M taps): 0.70 ms
-// against 0.77 without both; 100,000 points of 8 x 8 on 512^2: 0.069 against
-// 0.104 ms.  A private copy per wavefront (two workgroups per CU) took three
+// the next pair's first taps fly while a pair is added; a pair is tested
+// against the table's end once where all of it lies inside.  Measured,
+// 2,496,960 points of supports 8..48 in chunks of 306 on 2048^2 (330 M taps):
+// 0.65 ms against 0.77 without any of it; 100,000 points of 8 x 8 on 512^2:
+// 0.069 against 0.104 ms.  A private copy per wavefront (two workgroups per CU) took three
 // times as long, the taps of 2-8 slabs loaded together 4-70% more.  A tap
 // index past the table reads nothing and adds nothing.  add: the tile sums are
 // added to the grid's contents (otherwise the grid was zeroed and a tile
@@ -763,8 +764,10 @@ k_grid_tiles_f64(TiledDev d, const double2 *__restrict__ vis,
   // A pair as its lanes see it: rows lr, lr + rows, ... below h.
   struct Part {
     int lr, h, rows, tstep, cstep, cell;
+    int flip;   // the sign bit of a conjugated tap's imaginary part
+    bool in;    // all of the pair's taps lie in the table
     long long tap;
-    double vx, vy, sgn;
+    double vx, vy;
   };
   for_each_item(d, d.queue + Q_GRID, [&](const ItemRange &ir) {
     for (int q = threadIdx.x; q < CP; q += 64 * F64_WAVES) {
@@ -795,7 +798,8 @@ k_grid_tiles_f64(TiledDev d, const double2 *__restrict__ vis,
       p.cell = (r0 + lr) * LS + c0 + lc;
       p.tstep = p.rows * stride;
       p.cstep = p.rows * LS;
-      p.sgn = (px >> 30) & 1 ? -1.0 : 1.0;
+      p.flip = (px << 1) & 0x80000000;
+      p.in = py >= 0 && (long long)py + (long long)(p.h - 1) * stride + w <= n_taps;
       auto word = [&](double x) {
         const long long v = __double_as_longlong(x);
         return __longlong_as_double((long long)rl((int)(v >> 32), j) << 32 | (unsigned)rl((int)v, j));
@@ -804,8 +808,8 @@ k_grid_tiles_f64(TiledDev d, const double2 *__restrict__ vis,
       p.vy = word(mv.y);
       return p;
     };
-    auto load = [&](int row, int h, long long tap) {
-      return row < h && tap >= 0 && tap < n_taps ? taps[tap] : make_double2(0.0, 0.0);
+    auto first = [&](const Part &p) {
+      return p.in && p.lr < p.h ? taps[p.tap] : make_double2(0.0, 0.0);
     };
     if (npw > 0) fetch(0);
     for (int b = 0; b < npw; b += 64) {
@@ -814,23 +818,36 @@ k_grid_tiles_f64(TiledDev d, const double2 *__restrict__ vis,
       if (b + 64 < npw) fetch(b + 64);
       const int n = min(64, npw - b);
       Part p = part(0);
-      double2 t = load(p.lr, p.h, p.tap);
+      double2 t = first(p);
       for (int j = 0; j < n; j++) {
         // the next pair's first taps fly while this pair's are added
         const Part q = part(min(j + 1, n - 1));
-        const double2 t_next = load(q.lr, q.h, q.tap);
-        for (int row = p.lr; row < p.h;) {
-          if (p.tap >= 0 && p.tap < n_taps) {
-            const double ty = t.y * p.sgn;
-            const double pr = p.vx * t.x - p.vy * ty;
-            const double pi = p.vx * ty + p.vy * t.x;
-            __hip_atomic_fetch_add(&re[p.cell], pr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(&im[p.cell], pi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          }
-          row += p.rows;
+        const double2 t_next = first(q);
+        auto add_tap = [&]() {
+          const double ty = __hiloint2double(__double2hiint(t.y) ^ p.flip, __double2loint(t.y));
+          const double pr = p.vx * t.x - p.vy * ty;
+          const double pi = p.vx * ty + p.vy * t.x;
+          __hip_atomic_fetch_add(&re[p.cell], pr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          __hip_atomic_fetch_add(&im[p.cell], pi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           p.tap += p.tstep;
           p.cell += p.cstep;
-          t = load(row, p.h, p.tap);
+        };
+        if (p.in) {
+          for (int row = p.lr; row < p.h;) {
+            add_tap();
+            row += p.rows;
+            if (row < p.h) t = taps[p.tap];
+          }
+        } else {
+          for (int row = p.lr; row < p.h; row += p.rows) {
+            if (p.tap >= 0 && p.tap < n_taps) {
+              t = taps[p.tap];
+              add_tap();
+            } else {
+              p.tap += p.tstep;
+              p.cell += p.cstep;
+            }
+          }
         }
         p = q;
         t = t_next;
