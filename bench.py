@@ -82,7 +82,7 @@ def profiled(kernel: str) -> dict:
     """Counter figures per dispatch of `kernel` at the default headline
     workload, from the rocprofv3 summary committed under profiles/ (lines
     '<key> <kernel> <value>', the kernel named without spaces, e.g.
-    k_grid_tiles<32,3>: traffic_bytes = L2-to-memory bytes from the
+    k_grid_tiles<32,4>: traffic_bytes = L2-to-memory bytes from the
     per-request-size counters, valu_instr, salu_instr)."""
     p = ROOT / "profiles" / "wproj_tiled_traffic.md"
     out = {}
@@ -1127,12 +1127,14 @@ def main() -> int:
     # MALL, so never an HBM figure).
     t_dom = max(k_grid, k_degrid)
     # the kernels are templates on tile and wavefronts per workgroup (the
-    # plan's defaults: 3 gridding wavefronts at tile 32, else 4; 4 degridding)
+    # plan's defaults: 4 gridding, 4 degridding), the degridder of whole
+    # windows (tiles of up to 32 at support 64) on wavefronts only (8)
     if k_grid >= k_degrid:
-        dom, nw = "k_grid_tiles", args.waves or (3 if args.tile == 32 else 4)
+        kname = f"k_grid_tiles<{args.tile}, {args.waves or 4}>"
+    elif args.tile <= 32 and args.layout == "pairs":
+        kname = f"k_degrid_windows<{args.degrid_waves or 8}>"
     else:
-        dom, nw = "k_degrid_tiles", args.degrid_waves or 4
-    kname = f"{dom}<{args.tile}, {nw}>"
+        kname = f"k_degrid_tiles<{args.tile}, {args.degrid_waves or 4}>"
     sec = t_dom / 1e3
     slots = sec * CLOCK_GHZ * 1e9 * N_CU
     fp32_tf = 8 * taps / sec / 1e12

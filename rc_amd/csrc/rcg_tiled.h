@@ -11,7 +11,7 @@ namespace rcg {
 // (16384 ints = 64 KiB of LDS).
 constexpr int MAX_BIN_TILES = 16384;
 // Tiles of a whole plan (instances x tiles per instance) handled by the
-// three-kernel scan: 1024 segments of 1024 tiles.
+// scan in three kernels: 1024 segments of 1024 tiles.
 constexpr int MAX_PLAN_TILES = 1 << 20;
 // Error word bit: a pair did not fit the plan's pair buffer (a chunk
 // support above the plan's max_support).

@@ -1554,7 +1554,7 @@ rcg_status rcg::tiled_bin_records(rcg_tiled_plan *pl, hipStream_t st)
 namespace {
 
 // Counting sort of the plan's records into per-tile pair lists: LDS
-// histograms, three-kernel scan, LDS-ranked fill.
+// histograms, scan, LDS-ranked fill.
 rcg_status bin_passes(rcg_tiled_plan *pl, hipStream_t st)
 {
   TiledDev &d = pl->dev;
