@@ -112,6 +112,8 @@ def grid_plain_f64(geom: DeviceGeom, gcf: DeviceGCF, pg: torch.Tensor,
                    stream=None) -> torch.Tensor:
     if vis.dtype != torch.complex128 or gcf.data.dtype != torch.complex128:
         raise TypeError("FP64 path takes complex128 visibilities and taps")
+    if vis.numel() < geom.n:
+        raise ValueError(f"{vis.numel()} visibilities for {geom.n} points")
     if grid is None:
         grid = torch.empty((geom.grid_size, geom.grid_pitch), dtype=torch.complex128,
                            device=vis.device)

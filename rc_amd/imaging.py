@@ -81,8 +81,11 @@ class Imager:
     # -- building blocks -------------------------------------------------
     def grid(self, vis: torch.Tensor) -> torch.Tensor:
         if self.f64:
+            # (more visibilities than points: the first ones count)
             v = vis.to(self.cdtype).contiguous()
-            if self.plan is not None and v.numel() == self.geom.n:
+            if v.numel() > self.geom.n:
+                v = v.reshape(-1)[: self.geom.n]
+            if self.plan is not None:
                 return self.plan.grid_f64(self.gcf, v)
             return D.grid_plain_f64(self.geom, self.gcf, self.pg, v)
         return self.plan.grid(self.gcf, vis.to(self.cdtype).contiguous())
