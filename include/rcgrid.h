@@ -335,6 +335,15 @@ rcg_status rcg_degrid_tiled_f32(rcg_tiled_plan *plan, const rcg_gcf *gcf,
  * rcg_c128.  The gridder of the MS4 host-memory entry points. */
 rcg_status rcg_grid_tiled_f64(rcg_tiled_plan *plan, const rcg_gcf *gcf,
                               const rcg_c128 *vis, rcg_c128 *grid, void *stream);
+/* The same with work counters of the caller's, rcg_tiled_counter_bytes() of
+ * device memory that this call alone uses until it has run (its contents do
+ * not matter).  Calls with counters of their own only read the plan, so that
+ * they may run on several streams and from several threads at once; a call
+ * without them uses the plan's, one at a time. */
+size_t rcg_tiled_counter_bytes(void);
+rcg_status rcg_grid_tiled_f64_counters(rcg_tiled_plan *plan, const rcg_gcf *gcf,
+                                       const rcg_c128 *vis, rcg_c128 *grid,
+                                       void *counters, void *stream);
 /* FP64 degridding over a plan's pairs (binned as for rcg_grid_tiled_f64):
  * each visibility is the sum of the reference's products grid * tap in FP64
  * (scatter_gridder_w_dependent_dyn_1p.cpp:368-431, behind

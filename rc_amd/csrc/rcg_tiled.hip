@@ -1732,10 +1732,12 @@ rcg_status launch_grid_f64(const TiledDev &d, const double2 *v, const double2 *t
   return RCG_OK;
 }
 
+// queue: the eight work counters (null: the plan's).
 rcg_status grid_f64(rcg_tiled_plan *pl, const double2 *v, const double2 *t, long long nt,
-                    double2 *g, int add, hipStream_t st)
+                    double2 *g, int add, int *queue, hipStream_t st)
 {
   TiledDev d = pl->dev;
+  if (queue) d.queue = queue;
   if (d.layout != LAYOUT_PAIRS) {
     set_error(RCG_ERR_UNSUPPORTED, "FP64 tiled gridding needs a plan of RCG_LAYOUT_PAIRS");
     return RCG_ERR_UNSUPPORTED;
@@ -1885,8 +1887,21 @@ extern "C" rcg_status rcg_degrid_tiled_f64(rcg_tiled_plan *pl, const rcg_gcf *gc
                     reinterpret_cast<double2 *>(vis), (hipStream_t)stream);
 }
 
+static_assert(Q_GRID == 0, "a caller's counters are the gridder's");
+extern "C" size_t rcg_tiled_counter_bytes(void)
+{
+  return (size_t)8 * QUEUE_STRIDE * sizeof(int);
+}
+
 extern "C" rcg_status rcg_grid_tiled_f64(rcg_tiled_plan *pl, const rcg_gcf *gcf,
                                          const rcg_c128 *vis, rcg_c128 *grid, void *stream)
+{
+  return rcg_grid_tiled_f64_counters(pl, gcf, vis, grid, nullptr, stream);
+}
+
+extern "C" rcg_status rcg_grid_tiled_f64_counters(rcg_tiled_plan *pl, const rcg_gcf *gcf,
+                                                  const rcg_c128 *vis, rcg_c128 *grid,
+                                                  void *counters, void *stream)
 {
   clear_error();
   if (!pl || !gcf || !vis || !grid) {
@@ -1901,7 +1916,8 @@ extern "C" rcg_status rcg_grid_tiled_f64(rcg_tiled_plan *pl, const rcg_gcf *gcf,
   }
   return grid_f64(pl, reinterpret_cast<const double2 *>(vis),
                   reinterpret_cast<const double2 *>(gcf->data), gcf->n_taps,
-                  reinterpret_cast<double2 *>(grid), 0, (hipStream_t)stream);
+                  reinterpret_cast<double2 *>(grid), 0, static_cast<int *>(counters),
+                  (hipStream_t)stream);
 }
 
 rcg_status rcg::tiled_grid_f64_add(rcg_tiled_plan *pl, const double2 *taps, long long n_taps,
@@ -1911,7 +1927,7 @@ rcg_status rcg::tiled_grid_f64_add(rcg_tiled_plan *pl, const double2 *taps, long
     set_error(RCG_ERR_ARG, "tiled FP64 gridding: empty tap table");
     return RCG_ERR_ARG;
   }
-  return grid_f64(pl, vis, taps, n_taps, grid, 1, st);
+  return grid_f64(pl, vis, taps, n_taps, grid, 1, nullptr, st);
 }
 
 extern "C" rcg_status rcg_tiled_stats(rcg_tiled_plan *pl, unsigned long long *taps,

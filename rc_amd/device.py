@@ -236,10 +236,11 @@ class TiledPlan(_lib.Handle):
         return grid
 
     def grid_f64(self, gcf: DeviceGCF, vis: torch.Tensor, grid: torch.Tensor | None = None,
-                 stream=None) -> torch.Tensor:
+                 stream=None, own_counters: bool = False) -> torch.Tensor:
         """FP64 gridding over the plan's pairs (rcg_grid_tiled_f64): complex128
         taps (the plan binned with a table of the same layout), visibilities
-        and grid."""
+        and grid.  Calls with work counters of their own (own_counters) may
+        run on several streams at once; the others share the plan's."""
         if gcf.data.dtype != torch.complex128:
             raise TypeError("FP64 gridding takes complex128 taps")
         if vis.dtype != torch.complex128:
@@ -252,9 +253,16 @@ class TiledPlan(_lib.Handle):
                 not grid.is_contiguous():
             raise ValueError(f"grid must be a contiguous complex128 {self.grid_shape} tensor")
         t = gcf.struct()
-        _lib.check(_lib.lib().rcg_grid_tiled_f64(self._h, C.byref(t), vis.data_ptr(),
-                                                 grid.data_ptr(), _stream(stream)),
-                   "rcg_grid_tiled_f64")
+        counters = None
+        if own_counters:
+            counters = torch.empty(int(_lib.lib().rcg_tiled_counter_bytes()), dtype=torch.uint8,
+                                   device=vis.device)
+            if stream is not None:
+                counters.record_stream(stream)
+        _lib.check(_lib.lib().rcg_grid_tiled_f64_counters(
+            self._h, C.byref(t), vis.data_ptr(), grid.data_ptr(),
+            None if counters is None else counters.data_ptr(), _stream(stream)),
+            "rcg_grid_tiled_f64")
         return grid
 
     def degrid_f64(self, gcf: DeviceGCF, grid: torch.Tensor, vis: torch.Tensor | None = None,

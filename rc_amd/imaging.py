@@ -86,7 +86,9 @@ class Imager:
             if v.numel() > self.geom.n:
                 v = v.reshape(-1)[: self.geom.n]
             if self.plan is not None:
-                return self.plan.grid_f64(self.gcf, v)
+                # counters of the call's own: calls on several streams and
+                # threads share the plan and only read it
+                return self.plan.grid_f64(self.gcf, v, own_counters=True)
             return D.grid_plain_f64(self.geom, self.gcf, self.pg, v)
         return self.plan.grid(self.gcf, vis.to(self.cdtype).contiguous())
 
