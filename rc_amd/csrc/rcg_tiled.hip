@@ -1461,6 +1461,9 @@ rcg_status create_plan(const rcg_geom *geoms, int n_inst, int tile, int chunk, i
     e = hipMemcpy(pl->geoms_dev, head.data(), head.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     rcg_tiled_plan_destroy(pl);
+    // a caller that goes on without the plan checks its launches: they would
+    // report this error again
+    (void)hipGetLastError();
     set_error(RCG_ERR_NOMEM, "plan set-up failed: %s", hipGetErrorString(e));
     return RCG_ERR_NOMEM;
   }
