@@ -625,9 +625,9 @@ extern "C" void deconvolve(double *mod_p, double *res_p, double *psf_p, int siz,
   hipStream_t st = nullptr;
   void *dm = nullptr, *dr = nullptr, *dp = nullptr, *ds = nullptr;
   if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&dm, bytes) != hipSuccess || hipMalloc(&dr, bytes) != hipSuccess ||
-      hipMalloc(&dp, bytes) != hipSuccess ||
-      hipMalloc(&ds, rcg_hogbom_scratch_bytes()) != hipSuccess) {
+      dev_malloc(&dm, bytes) != hipSuccess || dev_malloc(&dr, bytes) != hipSuccess ||
+      dev_malloc(&dp, bytes) != hipSuccess ||
+      dev_malloc(&ds, rcg_hogbom_scratch_bytes()) != hipSuccess) {
     set_error(RCG_ERR_NOMEM, "deconvolve: device buffers");
   } else if (hipMemcpyAsync(dr, res_p, bytes, hipMemcpyHostToDevice, st) != hipSuccess ||
              hipMemcpyAsync(dp, psf_p, bytes, hipMemcpyHostToDevice, st) != hipSuccess) {

@@ -195,7 +195,7 @@ extern "C" rcg_status rcg_fft_plan_create(int sign, int f64, int size, int pitch
   }
   hipError_t e = hipSuccess;
   if (p->work_bytes) {
-    e = hipMalloc(&p->work, p->work_bytes);
+    e = dev_malloc(&p->work, p->work_bytes);
     if (e == hipSuccess)
       rs = rocfft_execution_info_set_work_buffer(p->info, p->work, p->work_bytes);
   }
@@ -203,7 +203,7 @@ extern "C" rcg_status rcg_fft_plan_create(int sign, int f64, int size, int pitch
     // real scratch [size][size] and complex scratch [size][size/2+1]
     const size_t elem = f64 ? 8 : 4;
     const size_t bytes = n * n * elem + n * (n / 2 + 1) * 2 * elem;
-    e = hipMalloc(&p->scratch, bytes);
+    e = dev_malloc(&p->scratch, bytes);
   }
   if (e != hipSuccess || rs != rocfft_status_success) {
     rcg_fft_plan_destroy(p);
@@ -323,7 +323,7 @@ extern "C" void *fft_inplace_even(void *plan, int sign, void *data, int size, in
   hipStream_t st = nullptr;
   void *d = nullptr;
   if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&d, bytes) != hipSuccess) {
+      dev_malloc(&d, bytes) != hipSuccess) {
     set_error(RCG_ERR_NOMEM, "fft_inplace_even: device buffers");
     if (st) (void)hipStreamDestroy(st);
     return p;

@@ -35,7 +35,7 @@ namespace {
 struct DevBuf {
   void *p = nullptr;
   ~DevBuf() { if (p) (void)hipFree(p); }
-  hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 16); }
+  hipError_t alloc(size_t bytes) { return dev_malloc(&p, bytes ? bytes : 16); }
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 

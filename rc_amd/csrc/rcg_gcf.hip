@@ -377,9 +377,9 @@ rcg_status gen_arena(rcg_gcf_gen *g)
 {
   if (g->fft) return RCG_OK;
   const size_t bytes = (size_t)g->L * g->pitch * sizeof(double2);
-  if ((!g->arena && hipMalloc(reinterpret_cast<void **>(&g->arena), bytes) != hipSuccess) ||
+  if ((!g->arena && dev_malloc(reinterpret_cast<void **>(&g->arena), bytes) != hipSuccess) ||
       (!g->sums &&
-       hipMalloc(reinterpret_cast<void **>(&g->sums), 64 * sizeof(double)) != hipSuccess)) {
+       dev_malloc(reinterpret_cast<void **>(&g->sums), 64 * sizeof(double)) != hipSuccess)) {
     set_error(RCG_ERR_NOMEM, "rcg_gcf_gen: device arena of %zu bytes", bytes);
     return RCG_ERR_NOMEM;
   }
@@ -541,7 +541,7 @@ extern "C" void *mkGCFLayer(void *p, rcg_c128 dst[], rcg_c128 *table[], rcg_c128
   hipStream_t st = nullptr;
   void *d = nullptr;
   if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&d, bytes) != hipSuccess) {
+      dev_malloc(&d, bytes) != hipSuccess) {
     set_error(RCG_ERR_NOMEM, "mkGCFLayer: device buffers");
   } else if (rcg_gcf_gen_layer(g, d, 1, support, t2, w, t_pad_quirk, st) == RCG_OK) {
     if (hipMemcpyAsync(dst, d, bytes, hipMemcpyDeviceToHost, st) != hipSuccess ||
@@ -567,10 +567,10 @@ extern "C" void calcAccums(const rcg_double3 uvw[], double sums[], int npts[], d
   void *du = nullptr, *ds = nullptr, *dn = nullptr, *de = nullptr;
   const size_t ub = (size_t)numDataPoints * sizeof(rcg_double3);
   if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&du, ub ? ub : 1) != hipSuccess ||
-      hipMalloc(&ds, numOfWPlanes * sizeof(double)) != hipSuccess ||
-      hipMalloc(&dn, numOfWPlanes * sizeof(int)) != hipSuccess ||
-      hipMalloc(&de, sizeof(int)) != hipSuccess) {
+      dev_malloc(&du, ub ? ub : 1) != hipSuccess ||
+      dev_malloc(&ds, numOfWPlanes * sizeof(double)) != hipSuccess ||
+      dev_malloc(&dn, numOfWPlanes * sizeof(int)) != hipSuccess ||
+      dev_malloc(&de, sizeof(int)) != hipSuccess) {
     set_error(RCG_ERR_NOMEM, "calcAccums: device buffers");
   } else if ((ub && hipMemcpyAsync(du, uvw, ub, hipMemcpyHostToDevice, st) != hipSuccess)) {
     set_error(RCG_ERR_HIP, "calcAccums: copy in");

@@ -222,7 +222,7 @@ hipError_t to_device(const buffer_t *b, bool gpu_mode, bool upload, hipStream_t 
     return hipSuccess;
   }
   const size_t bytes = (size_t)span_of(b) * sizeof(double);
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->p), bytes);
+  hipError_t e = dev_malloc(reinterpret_cast<void **>(&d->p), bytes);
   if (e != hipSuccess) {
     d->p = nullptr;
     return e;
@@ -298,7 +298,7 @@ int scatter_tiled(double scale, int grid_size, int margin, const buffer_t *vis,
   clear_error();
   (void)hipGetLastError();  // a failed plan allocation leaves its error behind
   if (!h.p) return 0;
-  if (hipMalloc(reinterpret_cast<void **>(&h.v2), (size_t)n * sizeof(double2)) != hipSuccess) {
+  if (dev_malloc(reinterpret_cast<void **>(&h.v2), (size_t)n * sizeof(double2)) != hipSuccess) {
     h.v2 = nullptr;
     (void)hipGetLastError();
     return 0;
@@ -612,10 +612,10 @@ int nv_grid_host(const char *who, double scale, double *out, const double *pos, 
   int rc = 0;
   PlanHold plan;
   if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&dp), pbytes) != hipSuccess ||
-      (!shared && hipMalloc(reinterpret_cast<void **>(&dv), vbytes) != hipSuccess) ||
-      hipMalloc(reinterpret_cast<void **>(&dg), gbytes) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&dout), obytes) != hipSuccess) {
+      dev_malloc(reinterpret_cast<void **>(&dp), pbytes) != hipSuccess ||
+      (!shared && dev_malloc(reinterpret_cast<void **>(&dv), vbytes) != hipSuccess) ||
+      dev_malloc(reinterpret_cast<void **>(&dg), gbytes) != hipSuccess ||
+      dev_malloc(reinterpret_cast<void **>(&dout), obytes) != hipSuccess) {
     set_error(RCG_ERR_NOMEM, "%s: device buffers", who);
     rc = -1;
   } else {
@@ -655,7 +655,7 @@ int nv_grid_host(const char *who, double scale, double *out, const double *pos, 
       clear_error();
       (void)hipGetLastError();  // a failed plan allocation leaves its error behind
       if (plan.p &&
-          hipMalloc(reinterpret_cast<void **>(&plan.v2), (size_t)n * sizeof(double2)) ==
+          dev_malloc(reinterpret_cast<void **>(&plan.v2), (size_t)n * sizeof(double2)) ==
               hipSuccess) {
         hipLaunchKernelGGL(k_nv_records, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
                            dp, ps, vals, vs, n, scale, img, plan.p->pg, plan.v2);
@@ -947,7 +947,7 @@ struct Glue {
     if (rc) return nullptr;
     const size_t bytes = (size_t)span_elems(b, dims) * sizeof(double);
     double *p = nullptr;
-    if (hipMalloc(reinterpret_cast<void **>(&p), bytes) != hipSuccess) {
+    if (dev_malloc(reinterpret_cast<void **>(&p), bytes) != hipSuccess) {
       fail(RCG_ERR_NOMEM);
       return nullptr;
     }
@@ -1158,7 +1158,7 @@ int defacet(buffer_t *facet, buffer_t *image)
   double *di = g.upload(image, 2, true);
   const long long pix = (long long)image->extent[0] * image->extent[1];
   unsigned long long *win = nullptr;
-  if (!g.rc && hipMalloc(reinterpret_cast<void **>(&win), pix * sizeof(unsigned long long)) !=
+  if (!g.rc && dev_malloc(reinterpret_cast<void **>(&win), pix * sizeof(unsigned long long)) !=
                    hipSuccess)
     g.fail(RCG_ERR_NOMEM);
   const G4 fg = g4_of(facet, 4), og = g4_of(image, 2);

@@ -42,6 +42,10 @@ inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 rcg_status check_geom(const rcg_geom *g);
 rcg_status check_gcf(const rcg_gcf *t);
 
+// hipMalloc for the whole library: an allocation that fails is tried again
+// without what the pool keeps, and leaves no HIP error behind.
+hipError_t dev_malloc(void **p, size_t bytes);
+
 // Device memory and streams kept between calls (rcg_pool.hip).  A block or
 // stream goes back only when nothing on the device uses it any more.
 hipError_t pool_get(void **p, size_t bytes);

@@ -294,7 +294,7 @@ struct DevMem {
   {
     if (p) (void)hipFree(p);
   }
-  hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 16); }
+  hipError_t alloc(size_t bytes) { return rcg::dev_malloc(&p, bytes ? bytes : 16); }
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 

@@ -7,7 +7,7 @@
 // comes back to the pool only when its call has waited for its stream, so it
 // is idle and may go to any thread and stream next.  At most POOL_BYTES are
 // kept per process; a block that does not fit is freed, and so is all that is
-// kept when an allocation fails and in rcg_shutdown.  The state is never
+// kept when an allocation of the library fails and in rcg_shutdown.  The state is never
 // destroyed, so nothing calls HIP when the process ends.
 #include <algorithm>
 #include <atomic>
@@ -70,7 +70,30 @@ void drop_all(Pool &p)
   p.kept = 0;
 }
 
+// p.mu is held.
+hipError_t malloc_or_drop(Pool &p, void **out, size_t bytes)
+{
+  hipError_t e = hipMalloc(out, bytes);
+  if (e != hipSuccess && p.kept) {
+    (void)hipGetLastError();
+    drop_all(p);
+    e = hipMalloc(out, bytes);
+  }
+  if (e != hipSuccess) {
+    *out = nullptr;
+    (void)hipGetLastError();
+  }
+  return e;
+}
+
 }  // namespace
+
+hipError_t dev_malloc(void **out, size_t bytes)
+{
+  Pool &p = pool();
+  std::lock_guard<std::mutex> lk(p.mu);
+  return malloc_or_drop(p, out, bytes);
+}
 
 hipError_t pool_get(void **out, size_t bytes)
 {
@@ -89,12 +112,7 @@ hipError_t pool_get(void **out, size_t bytes)
     if (f->second.empty()) p.free.erase(f);
     return hipSuccess;
   }
-  e = hipMalloc(out, size);
-  if (e != hipSuccess && p.kept) {
-    (void)hipGetLastError();
-    drop_all(p);
-    e = hipMalloc(out, size);
-  }
+  e = malloc_or_drop(p, out, size);
   if (e == hipSuccess) p.out[*out] = {dev, size};
   return e;
 }

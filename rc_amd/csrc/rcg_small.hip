@@ -206,7 +206,7 @@ namespace {
 struct DevBuf {
   void *p = nullptr;
   ~DevBuf() { if (p) (void)hipFree(p); }
-  hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 16); }
+  hipError_t alloc(size_t bytes) { return dev_malloc(&p, bytes ? bytes : 16); }
 };
 
 bool grid_dims_ok(int pitch, int size)

@@ -1159,7 +1159,7 @@ hipError_t dalloc(T **p, size_t n, bool pooled)
 {
   void **v = reinterpret_cast<void **>(p);
   const size_t bytes = (n ? n : 1) * sizeof(T);
-  return pooled ? pool_get(v, bytes) : hipMalloc(v, bytes);
+  return pooled ? pool_get(v, bytes) : dev_malloc(v, bytes);
 }
 
 // Persistent workgroups of a kernel: resident workgroups per CU x CUs,
@@ -1648,7 +1648,7 @@ extern "C" rcg_status rcg_tiled_compensated(rcg_tiled_plan *pl, int enable)
   }
   if (enable && !pl->lo) {
     const size_t cells = (size_t)pl->dev.gstride * pl->dev.n_inst;
-    if (hipMalloc(reinterpret_cast<void **>(&pl->lo), cells * sizeof(float2)) != hipSuccess) {
+    if (dev_malloc(reinterpret_cast<void **>(&pl->lo), cells * sizeof(float2)) != hipSuccess) {
       pl->lo = nullptr;
       set_error(RCG_ERR_NOMEM, "rcg_tiled_compensated: %zu cells", cells);
       return RCG_ERR_NOMEM;
