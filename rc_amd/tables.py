@@ -20,6 +20,12 @@ import numpy as np
 OVER = 8  # MS4/kernel/common/metrix.h:5
 
 
+class _Pointer(C.c_void_p):
+    """An address that holds the array it points into."""
+
+    array = None
+
+
 @dataclass
 class GCFTable:
     """A GCF table in host memory.
@@ -98,7 +104,9 @@ class GCFTable:
     def pointer_tables(self):
         """(centred layer-pointer table, centred support pointer) as c_void_p.
 
-        The arrays behind them stay alive as long as this object does.
+        The arrays behind them stay alive as long as the pointer returned
+        (calls of several threads on one table have arrays of their own), the
+        last call's also as long as this object.
         """
         item = self.data.dtype.itemsize
         base = self.data.ctypes.data
@@ -106,8 +114,10 @@ class GCFTable:
             *[base + int(o) * item for o in self.layer_off])
         supps = np.ascontiguousarray(self.supps, np.int32)
         self._keep[:] = [ptrs, supps]
-        gcf_c = C.c_void_p(C.addressof(ptrs) + self.center * C.sizeof(C.c_void_p))
-        sup_c = C.c_void_p(supps.ctypes.data + self.max_w_plane * 4)
+        gcf_c = _Pointer(C.addressof(ptrs) + self.center * C.sizeof(C.c_void_p))
+        gcf_c.array = ptrs
+        sup_c = _Pointer(supps.ctypes.data + self.max_w_plane * 4)
+        sup_c.array = supps
         return gcf_c, sup_c
 
 
