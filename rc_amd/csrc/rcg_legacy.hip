@@ -82,19 +82,28 @@ struct LegacyArgs {
 // (rcg_legacy_grid_path).
 thread_local int t_last_path = RCG_PATH_NONE;
 
+size_t grid_cells(const LegacyArgs &a)
+{
+  return (a.size > 0 && a.pitch > 0) ? (size_t)a.size * a.pitch : 0;
+}
+
+void zero_result(const LegacyArgs &a)
+{
+  if (!a.degrid) {
+    const size_t gcells = grid_cells(a);
+    if (a.grid_out && gcells) memset(a.grid_out, 0, gcells * sizeof(rcg_c128));
+  } else if (a.vis_out && a.ts_ch > 0) {
+    for (int bl = 0; bl < a.baselines; bl++)
+      if (a.vis_out[bl]) memset(a.vis_out[bl], 0, (size_t)a.ts_ch * sizeof(rcg_c128));
+  }
+}
+
 ull legacy_call(const LegacyArgs &a)
 {
   clear_error();
   t_last_path = RCG_PATH_NONE;
-  const size_t gcells = (a.size > 0 && a.pitch > 0) ? (size_t)a.size * a.pitch : 0;
-  auto zero_outputs = [&]() {
-    if (!a.degrid) {
-      if (a.grid_out && gcells) memset(a.grid_out, 0, gcells * sizeof(rcg_c128));
-    } else if (a.vis_out && a.ts_ch > 0) {
-      for (int bl = 0; bl < a.baselines; bl++)
-        if (a.vis_out[bl]) memset(a.vis_out[bl], 0, (size_t)a.ts_ch * sizeof(rcg_c128));
-    }
-  };
+  const size_t gcells = grid_cells(a);
+  auto zero_outputs = [&]() { zero_result(a); };
   // host staging must outlive the copies queued from it, also where the call
   // ends early
   hipStream_t st = nullptr;
@@ -383,6 +392,18 @@ ull legacy_call(const LegacyArgs &a)
   return counts.taps;
 }
 
+// A C caller gets an error for what the call's host containers throw.
+ull legacy_entry(const LegacyArgs &a)
+{
+  try {
+    return legacy_call(a);
+  } catch (const std::bad_alloc &) {
+    zero_result(a);
+    set_error(RCG_ERR_NOMEM, "no host memory for the call's tables");
+    return 0;
+  }
+}
+
 }  // namespace
 }  // namespace rcg
 
@@ -399,7 +420,7 @@ ull legacy_call(const LegacyArgs &a)
     a.grid_in = nullptr; a.gcf = gcf; a.uvw = uvw; a.vis_in = vis;            \
     a.vis_out = nullptr; a.ts_ch = ts_ch; a.pitch = grid_pitch;               \
     a.size = grid_size; a.gcf_supps = gcf_supps;                              \
-    return rcg::legacy_call(a);                                               \
+    return rcg::legacy_entry(a);                                              \
   }
 
 #define RCG_LEGACY_DEGRID(name, is_half)                                       \
@@ -415,7 +436,7 @@ ull legacy_call(const LegacyArgs &a)
     a.grid_in = grid; a.gcf = gcf; a.uvw = uvw; a.vis_in = nullptr;           \
     a.vis_out = vis; a.ts_ch = ts_ch; a.pitch = grid_pitch;                   \
     a.size = grid_size; a.gcf_supps = gcf_supps;                              \
-    return rcg::legacy_call(a);                                               \
+    return rcg::legacy_entry(a);                                              \
   }
 
 RCG_LEGACY_GRID(gridKernelCPUFullGCF, false)

@@ -8,7 +8,9 @@
 // is idle and may go to any thread and stream next.  At most POOL_BYTES are
 // kept per process; a block that does not fit is freed, and so is all that is
 // kept when an allocation of the library fails and in rcg_shutdown.  The state is never
-// destroyed, so nothing calls HIP when the process ends.
+// destroyed, so nothing calls HIP when the process ends.  Nothing here throws
+// (callers are C entry points, destructors and threads): without host memory
+// for its lists the pool allocates nothing, or keeps nothing.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -70,6 +72,16 @@ void drop_all(Pool &p)
   p.kept = 0;
 }
 
+bool note_out(Pool &p, void *b, std::pair<int, size_t> key) noexcept
+{
+  try {
+    p.out[b] = key;
+    return true;
+  } catch (...) {
+    return false;
+  }
+}
+
 // p.mu is held.
 hipError_t malloc_or_drop(Pool &p, void **out, size_t bytes)
 {
@@ -105,15 +117,20 @@ hipError_t pool_get(void **out, size_t bytes)
   std::lock_guard<std::mutex> lk(p.mu);
   auto f = p.free.lower_bound({dev, size});
   if (f != p.free.end() && f->first.first == dev && f->first.second <= size + size / 4) {
-    *out = f->second.back();
+    void *b = f->second.back();
+    if (!note_out(p, b, f->first)) return hipErrorOutOfMemory;
+    *out = b;
     f->second.pop_back();
     p.kept -= f->first.second;
-    p.out[*out] = f->first;
     if (f->second.empty()) p.free.erase(f);
     return hipSuccess;
   }
   e = malloc_or_drop(p, out, size);
-  if (e == hipSuccess) p.out[*out] = {dev, size};
+  if (e == hipSuccess && !note_out(p, *out, {dev, size})) {
+    (void)hipFree(*out);
+    *out = nullptr;
+    e = hipErrorOutOfMemory;
+  }
   return e;
 }
 
@@ -125,12 +142,18 @@ void pool_put(void *b)
   const auto o = p.out.find(b);
   const auto key = o->second;
   p.out.erase(o);
-  if (p.kept + key.second > POOL_BYTES) {
-    (void)hipFree(b);
-    return;
+  if (p.kept + key.second <= POOL_BYTES) {
+    auto f = p.free.end();
+    try {
+      f = p.free.try_emplace(key).first;
+      f->second.push_back(b);
+      p.kept += key.second;
+      return;
+    } catch (...) {
+      if (f != p.free.end() && f->second.empty()) p.free.erase(f);
+    }
   }
-  p.free[key].push_back(b);
-  p.kept += key.second;
+  (void)hipFree(b);
 }
 
 hipError_t pool_stream(hipStream_t *st)
@@ -141,10 +164,10 @@ hipError_t pool_stream(hipStream_t *st)
   if (e != hipSuccess) return e;
   {
     std::lock_guard<std::mutex> lk(p.mu);
-    auto &s = p.streams[dev];
-    if (!s.empty()) {
-      *st = s.back();
-      s.pop_back();
+    const auto s = p.streams.find(dev);
+    if (s != p.streams.end() && !s->second.empty()) {
+      *st = s->second.back();
+      s->second.pop_back();
       return hipSuccess;
     }
   }
@@ -157,10 +180,13 @@ void pool_stream_put(hipStream_t st)
   int dev = 0;
   if (hipGetDevice(&dev) == hipSuccess) {
     std::lock_guard<std::mutex> lk(p.mu);
-    auto &s = p.streams[dev];
-    if (s.size() < POOL_STREAMS) {
-      s.push_back(st);
-      return;
+    try {
+      auto &s = p.streams[dev];
+      if (s.size() < POOL_STREAMS) {
+        s.push_back(st);
+        return;
+      }
+    } catch (...) {
     }
   }
   (void)hipStreamDestroy(st);
@@ -199,9 +225,12 @@ void pin_put(void *b)
   Pool &p = pool();
   {
     std::lock_guard<std::mutex> lk(p.mu);
-    if (p.pins.size() < POOL_PINS) {
-      p.pins.push_back(b);
-      return;
+    try {
+      if (p.pins.size() < POOL_PINS) {
+        p.pins.push_back(b);
+        return;
+      }
+    } catch (...) {
     }
   }
   (void)hipHostFree(b);

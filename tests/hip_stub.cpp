@@ -49,6 +49,7 @@ size_t stub_live() { return live; }
 size_t stub_frees() { return n_free; }
 long stub_launches() { return launches; }
 void stub_fail_new(int n) { fail_new = n; }
+int stub_new_left() { return fail_new; }
 
 int hipMalloc(void **p, size_t bytes)
 {

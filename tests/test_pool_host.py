@@ -56,3 +56,34 @@ assert stub.stub_live() == 0           # nothing kept, nothing lost
 print("ok")
 """)
     assert out.split() == ["ok"]
+
+
+def test_calls_without_host_memory(tmp_path):
+    """Every C++ allocation of a call in turn fails: the call ends with an
+    error or does without, nothing is lost, and the next call works.  (An
+    exception that left a C entry point, a destructor or a thread would end
+    the process.)"""
+    out = hipstub.run(tmp_path, KEEP + """
+h.rcg_shutdown()
+assert stub.stub_live() == 0
+failed = 0
+for n in range(1, 400):
+    stub.stub_fail_new(n)
+    try:
+        ms4.grid(vc, gcf, 64)
+    except _lib.RcgError:
+        assert h.rcg_last_error() in (2, 3)
+        failed += 1
+    left = stub.stub_new_left()        # 0: the n-th allocation was reached
+    stub.stub_fail_new(0)
+    ms4.grid(vc, gcf, 64)
+    assert stub.stub_live() == kept
+    if n % 2:
+        h.rcg_shutdown()
+        assert stub.stub_live() == 0
+    if left:
+        break
+assert 1 <= failed < n < 399, (failed, n)
+print("ok")
+""")
+    assert out.split() == ["ok"]
