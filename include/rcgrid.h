@@ -463,15 +463,19 @@ rcg_status rcg_fft_plan_destroy(rcg_fft_plan *plan);
 rcg_status rcg_shutdown(void);
 
 /* GCF generation on device memory (the reference's mkGCFLayer and
- * calcAccums, GCF.cpp:16-219).  A generator of the FP64 arena with side 8
- * max_support and row pitch 8 max_support + src_pad (held in memory only for
- * pad_quirk, whose sums walk it);
+ * calcAccums, GCF.cpp:16-219).  A generator owns the FP64 arena with side 8
+ * max_support and row pitch 8 max_support + src_pad, and its rocFFT plan,
+ * for pad_quirk, whose sums walk it; rcg_gcf_gen_create_ex with arena 0 puts
+ * them off to the first pad_quirk call (which then allocates, so that it
+ * cannot be captured in a graph);
  * rcg_gcf_gen_layer writes one plane's 64 layers [8][8][support][support]
  * to dst (complex128 if f64, else complex64).  rcg_calc_accums: device uvw,
  * sums (double) and npts (int) of n_planes entries, err_dev one device int
  * (bit 0: points outside the planes, skipped). */
 typedef struct rcg_gcf_gen rcg_gcf_gen;
 rcg_status rcg_gcf_gen_create(int max_support, int src_pad, rcg_gcf_gen **gen);
+rcg_status rcg_gcf_gen_create_ex(int max_support, int src_pad, int arena,
+                                 rcg_gcf_gen **gen);
 rcg_status rcg_gcf_gen_layer(rcg_gcf_gen *gen, void *dst, int f64, int support,
                              double t2, double w, int pad_quirk, void *stream);
 /* rcg_gcf_gen_layer for n planes (host arrays): plane k's layers of

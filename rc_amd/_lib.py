@@ -156,6 +156,7 @@ SIGNATURES: dict[str, tuple] = {
     "rcg_flow_binner": (C.c_int, [vp, C.c_int, C.c_int, vp, C.c_int, vp, vp, vp, vp, vp]),
     # GCF generation (device)
     "rcg_gcf_gen_create": (C.c_int, [C.c_int, C.c_int, C.POINTER(vp)]),
+    "rcg_gcf_gen_create_ex": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(vp)]),
     "rcg_gcf_gen_layer": (C.c_int, [vp, vp, C.c_int, C.c_int, C.c_double, C.c_double, C.c_int,
                                     vp]),
     "rcg_gcf_gen_layers": (C.c_int, [vp, vp, C.c_int, C.c_int, vp, vp, C.c_double, vp, C.c_int,

@@ -31,8 +31,8 @@
 // (k_gcf_layers).  The sum over a sub-lattice needs no samples: the sum over
 // its max_support^2 places of E's products is max_support^2 for the cell
 // a = b = R, where the screen is 1, and 0 for every other.  With pad_quirk the
-// sums need the whole padded arena: screen, rocFFT (rcg_fft plan, made on
-// first use), 64 workgroups for the sums, one kernel for the window.
+// sums need the whole padded arena: screen, rocFFT (rcg_fft plan), 64
+// workgroups for the sums, one kernel for the window.
 // calcAccums uses per-workgroup LDS histograms and one FP64 atomic per
 // touched plane per workgroup.
 #include <algorithm>
@@ -47,7 +47,8 @@ constexpr int ACC_MAX_PLANES = 8192;
 struct rcg_gcf_gen {
   int max_support, src_pad, L, pitch;
   bool held = false;         // counted as a user of the FFT library state
-  // pad_quirk only, made on first use
+  // pad_quirk only: made with the generator, or on first use where its maker
+  // asked for that (rcg_gcf_gen_create_ex)
   double2 *arena = nullptr;  // L rows x pitch complex
   double *sums = nullptr;    // 64 sub-lattice sums
   rcg_fft_plan *fft = nullptr;
@@ -346,7 +347,31 @@ extern "C" rcg_status rcg_gcf_gen_destroy(rcg_gcf_gen *g)
   return RCG_OK;
 }
 
+namespace {
+
+// The arena, sums and FFT plan of the pad_quirk path.
+rcg_status gen_arena(rcg_gcf_gen *g)
+{
+  if (g->fft) return RCG_OK;
+  const size_t bytes = (size_t)g->L * g->pitch * sizeof(double2);
+  if ((!g->arena && dev_malloc(reinterpret_cast<void **>(&g->arena), bytes) != hipSuccess) ||
+      (!g->sums &&
+       dev_malloc(reinterpret_cast<void **>(&g->sums), 64 * sizeof(double)) != hipSuccess)) {
+    set_error(RCG_ERR_NOMEM, "rcg_gcf_gen: device arena of %zu bytes", bytes);
+    return RCG_ERR_NOMEM;
+  }
+  return rcg_fft_plan_create(1, 1, g->L, g->pitch, &g->fft);
+}
+
+}  // namespace
+
 extern "C" rcg_status rcg_gcf_gen_create(int max_support, int src_pad, rcg_gcf_gen **out)
+{
+  return rcg_gcf_gen_create_ex(max_support, src_pad, 1, out);
+}
+
+extern "C" rcg_status rcg_gcf_gen_create_ex(int max_support, int src_pad, int arena,
+                                            rcg_gcf_gen **out)
 {
   clear_error();
   if (!out || max_support < 2 || max_support > MAX_SUPPORT || src_pad < 0 || src_pad > 4096) {
@@ -366,25 +391,16 @@ extern "C" rcg_status rcg_gcf_gen_create(int max_support, int src_pad, rcg_gcf_g
   g->pitch = g->L + src_pad;
   fft_hold(1);
   g->held = true;
+  const rcg_status s = arena ? gen_arena(g) : RCG_OK;
+  if (s != RCG_OK) {
+    rcg_gcf_gen_destroy(g);
+    return s;
+  }
   *out = g;
   return RCG_OK;
 }
 
 namespace {
-
-// The arena, sums and FFT plan of the pad_quirk path.
-rcg_status gen_arena(rcg_gcf_gen *g)
-{
-  if (g->fft) return RCG_OK;
-  const size_t bytes = (size_t)g->L * g->pitch * sizeof(double2);
-  if ((!g->arena && dev_malloc(reinterpret_cast<void **>(&g->arena), bytes) != hipSuccess) ||
-      (!g->sums &&
-       dev_malloc(reinterpret_cast<void **>(&g->sums), 64 * sizeof(double)) != hipSuccess)) {
-    set_error(RCG_ERR_NOMEM, "rcg_gcf_gen: device arena of %zu bytes", bytes);
-    return RCG_ERR_NOMEM;
-  }
-  return rcg_fft_plan_create(1, 1, g->L, g->pitch, &g->fft);
-}
 
 rcg_status quirk_layer(rcg_gcf_gen *g, void *dst, int f64, int support, double t2, double w,
                        hipStream_t st)
@@ -536,7 +552,8 @@ extern "C" void *mkGCFLayer(void *p, rcg_c128 dst[], rcg_c128 *table[], rcg_c128
               g->max_support, g->src_pad);
     return p;
   }
-  if (!g && rcg_gcf_gen_create(max_support, src_pad, &g) != RCG_OK) return nullptr;
+  if (!g && rcg_gcf_gen_create_ex(max_support, src_pad, t_pad_quirk ? 1 : 0, &g) != RCG_OK)
+    return nullptr;
   const size_t bytes = 64ull * support * support * sizeof(rcg_c128);
   hipStream_t st = nullptr;
   void *d = nullptr;

@@ -20,12 +20,13 @@ from .tables import OVER
 
 
 class GCFGenerator(_lib.Handle):
-    """rcg_gcf_gen: FP64 arena and rocFFT plan for one max_support/src_pad."""
+    """rcg_gcf_gen for one max_support/src_pad.  arena: with the FP64 arena and
+    rocFFT plan that pad_quirk needs; without, its first use makes them."""
 
-    def __init__(self, max_support: int, src_pad: int = 4):
+    def __init__(self, max_support: int, src_pad: int = 4, arena: bool = True):
         h = C.c_void_p()
-        _lib.check(_lib.lib().rcg_gcf_gen_create(max_support, src_pad, C.byref(h)),
-                   "rcg_gcf_gen_create")
+        _lib.check(_lib.lib().rcg_gcf_gen_create_ex(max_support, src_pad, int(arena),
+                                                    C.byref(h)), "rcg_gcf_gen_create")
         self.max_support, self.src_pad = max_support, src_pad
         self._own(h)
 
@@ -118,7 +119,8 @@ def make_gcf(uvw: torch.Tensor, wstep: float, theta: float, min_size: int, growt
     offs = np.concatenate([[0], np.cumsum(lens)])
     dev = uvw.device
     data = torch.empty(int(offs[-1]), dtype=dtype, device=dev)
-    gen = GCFGenerator(max_size, src_pad)
+    # (the arena and its plan take milliseconds to make)
+    gen = GCFGenerator(max_size, src_pad, arena=pad_quirk)
     try:
         gen.layers(data, sup, offs[:-1:OVER * OVER], theta / 2.0, np.asarray(means) * theta,
                    pad_quirk, stream)

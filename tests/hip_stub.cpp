@@ -2,7 +2,7 @@
 // host code without a GPU.  Loaded before librcgrid.so (RTLD_GLOBAL), its
 // functions take the place of the runtime's: device memory is host memory
 // within a limit, streams do nothing, kernel launches are counted and not
-// run.  As in the runtime, a call that fails leaves its error for
+// run, rocFFT plans are empty.  As in the runtime, a call that fails leaves its error for
 // hipGetLastError, which clears it.
 #include <atomic>
 #include <cstdlib>
@@ -170,6 +170,33 @@ int hipGetLastError()
   return e;
 }
 const char *hipGetErrorString(int) { return "stub error"; }
+
+// rocFFT: plans of no content
+int rocfft_setup() { return OK; }
+int rocfft_cleanup() { return OK; }
+int rocfft_plan_create(void **p, int, int, int, size_t, const size_t *, size_t, void *)
+{
+  *p = malloc(1);
+  return OK;
+}
+int rocfft_plan_destroy(void *p)
+{
+  free(p);
+  return OK;
+}
+int rocfft_plan_description_create(void **p) { return rocfft_plan_create(p, 0, 0, 0, 0, nullptr, 0, nullptr); }
+int rocfft_plan_description_destroy(void *p) { return rocfft_plan_destroy(p); }
+int rocfft_plan_description_set_data_layout(...) { return OK; }
+int rocfft_execution_info_create(void **p) { return rocfft_plan_create(p, 0, 0, 0, 0, nullptr, 0, nullptr); }
+int rocfft_execution_info_destroy(void *p) { return rocfft_plan_destroy(p); }
+int rocfft_execution_info_set_stream(void *, void *) { return OK; }
+int rocfft_execution_info_set_work_buffer(void *, void *, size_t) { return OK; }
+int rocfft_plan_get_work_buffer_size(void *, size_t *n)
+{
+  *n = 4096;
+  return OK;
+}
+int rocfft_execute(void *, void **, void **, void *) { return OK; }
 
 }  // extern "C"
 
