@@ -27,7 +27,8 @@
 // only support^2 samples per sub-lattice are kept, so the transform is two
 // small matrix products, out = E X E^T with E[u][a] = exp(2 pi i (u - L/2)
 // (a - R) / L) (L = 8 max_support, R = max_support / 2, X the screen): FP64
-// matrix instructions on 16 x 16 blocks, one launch for all planes of a table
+// matrix instructions on 16 x 16 blocks, the terms of equal cells of X (which
+// is even in both coordinates) together, one launch for all planes of a table
 // (k_gcf_layers).  The sum over a sub-lattice needs no samples: the sum over
 // its max_support^2 places of E's products is max_support^2 for the cell
 // a = b = R, where the screen is 1, and 0 for every other.  With pad_quirk the
@@ -107,15 +108,15 @@ struct GcfPlanes {
 };
 
 constexpr int GCF_ROWS = 32;  // output rows of a workgroup
+constexpr int GCF_THREADS = 1024, GCF_WAVES = GCF_THREADS / 64;
 
-// LDS of k_gcf_layers: E's L roots of unity, Y (GCF_ROWS x max_support,
-// padded to whole blocks; a row one more than a multiple of 16 cells, so that
-// the 16 rows of an operand start in different banks, except where that would
-// not fit) and, where it fits, the
-// screen's quadrant (the screen is even in both coordinates).
+// LDS of k_gcf_layers: the L roots of unity, Y (GCF_ROWS x (R + 1), padded to
+// whole blocks; a row one more than a multiple of 16 cells, so that the 16
+// rows of an operand start in different banks) and, where it fits, the
+// screen's quadrant.
 __host__ __device__ inline int gcf_ypitch(int ms)
 {
-  return ((ms + 15) & ~15) + (ms > 240 ? 0 : 1);
+  return ((ms / 2 + 1 + 15) & ~15) + 1;
 }
 size_t gcf_lds(int ms, bool quad)
 {
@@ -126,31 +127,37 @@ constexpr size_t GCF_LDS = 160 * 1024;
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-// acc += A B on 16 x 16 blocks, four complex products deep: A's row lane % 16,
-// B's column lane % 16, term lane / 16; the result's column lane % 16, rows
+// acc += a b on 16 x 16 blocks, four products deep: A's row lane % 16, B's
+// column lane % 16, term lane / 16; the result's column lane % 16, rows
 // 4 i + lane / 16.
-__device__ __forceinline__ void mfma_c(d4 &re, d4 &im, double2 a, double2 b)
+__device__ __forceinline__ void mfma_d(d4 &acc, double a, double b)
 {
-  re = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, re, 0, 0, 0);
-  im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, im, 0, 0, 0);
-  re = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, re, 0, 0, 0);
-  im = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, im, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
 }
 
-// 32 rows u of one plane: Y = E X (each wavefront a share of the columns), then
-// Y E^T (each a share of the column blocks).  Output columns are taken in the
-// order (over_v, sv), so that 16 lanes write consecutive taps.  Bound by the
-// matrix units and, for small supports, by the screen and the roots, which
-// every workgroup computes (1089 + 512 sincos at max_support 64).  Measured
-// for planes -31..31 with supports 8..64 at max_support 64 (taps and sums):
+// 32 rows u of one plane: Y = E X, then Y E^T, each wavefront a share of the
+// blocks of 16 x 16.  X is even in both coordinates, and so is Y in its
+// second: the terms a and -a from the centre go together, with the real
+// coefficient 2 cos, over a = 0..R.  Of an even max_support the last, a = R,
+// stands for -R alone: coefficient exp(-i phi R), its imaginary part added
+// by itself.  Output columns are taken in the order (over_v, sv), so that 16
+// lanes write consecutive taps.  Bound by the matrix units and, for small
+// supports, by the screen and the roots, which every workgroup computes (1089
+// + 512 sincos at max_support 64).  One plane has few workgroups (64 at
+// support 256) and from max_support 100 on a CU holds one, so the workgroup is
+// as large as can be.  Measured, one plane of support = max_support 64 / 128 /
+// 256, and 63 planes of it: 31 / 85 / 288 us and 0.24 / 0.82 / 4.7 ms; with 512
+// threads 34 / 95 / 327 us, with 256 57 / 172 / 638; with all max_support^2
+// terms, complex coefficients and 256 threads 79 / 283 / 1099 us; by rocFFT
+// 65 / 122 / 302 us and, with the making of its plan, 6 / 12 / 23 ms.
 template <class T, bool QUAD>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(GCF_THREADS)
 k_gcf_layers(GcfPlanes pl, int ms, double t2, T *__restrict__ out)
 {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   double2 *root = reinterpret_cast<double2 *>(smem);
   double2 *Y = root + 8 * ms;
-  const int yp = gcf_ypitch(ms), R = ms / 2, L = 8 * ms;
+  const int yp = gcf_ypitch(ms), R = ms / 2, L = 8 * ms, even = 1 - (ms & 1);
   double2 *quad = Y + GCF_ROWS * yp;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, l4 = lane >> 4;
@@ -159,83 +166,88 @@ k_gcf_layers(GcfPlanes pl, int ms, double t2, T *__restrict__ out)
   const int S = pl.support[p];
   const double w = pl.w[p], normer = t2 / (double)R;
   T *dst = out + pl.off[p];
-  for (int k = threadIdx.x; k < L; k += 256) {
+  for (int k = threadIdx.x; k < L; k += GCF_THREADS) {
     double s, c;
     sincospi(2.0 * (double)k / (double)L, &s, &c);
     root[k] = make_double2(c, s);
   }
   if (QUAD) {
     const int qs = R + 1;
-    for (int k = threadIdx.x; k < qs * qs; k += 256)
+    for (int k = threadIdx.x; k < qs * qs; k += GCF_THREADS)
       quad[k] = screen_cell(k / qs, k % qs, normer, w);
   }
   __syncthreads();
-  auto screen = [&](int a, int b) {  // a, b in [0, ms), else 0
-    if (a >= ms || b >= ms) return make_double2(0.0, 0.0);
-    const int x = abs(a - R), y = abs(b - R);
-    return QUAD ? quad[x * (R + 1) + y] : screen_cell(x, y, normer, w);
+  auto screen = [&](int a, int b) {  // a, b in [0, R], else 0
+    if (a > R || b > R) return make_double2(0.0, 0.0);
+    return QUAD ? quad[a * (R + 1) + b] : screen_cell(a, b, normer, w);
   };
   auto mod = [&](int k) {  // into [0, L)
     k %= L;
     return k < 0 ? k + L : k;
   };
+  // coefficient of term a (root index e = u a mod L)
+  auto coef = [&](int a, int e) {
+    const double c = a > R ? 0.0 : root[e].x;
+    return a == 0 || (even && a == R) ? c : 2.0 * c;
+  };
   const int n8 = 8 * S;                           // output rows and columns
   const int start = (ms / 2 - S / 2) * GCF_OVER;  // of the window in the arena
   const int row0 = ((int)blockIdx.x - pl.first[p]) * GCF_ROWS;
-  // this lane's two A rows of E: index of exp(2 pi i (u - L/2)(a - R) / L) at
-  // a = l4, and its step for a + 4
-  int e0[2], de[2];
-  for (int h = 0; h < 2; h++) {
-    const int u = mod(start + min(row0 + 16 * h + l16, n8 - 1) - L / 2);
-    e0[h] = mod(u * (l4 - R));
-    de[h] = mod(4 * u);
-  }
-  for (int b0 = wave * 16; b0 < ms; b0 += 64) {
-    d4 re[2] = {}, im[2] = {};
-    int e[2] = {e0[0], e0[1]};
-    for (int a = l4; a < ms + l4; a += 4) {
-      const double2 x = screen(a, b0 + l16);  // 0 past ms
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        mfma_c(re[h], im[h], root[e[h]], x);
-        e[h] += de[h];
-        e[h] -= e[h] >= L ? L : 0;
-      }
+  // this wavefront's 16 of the rows, and its first block of 16 columns
+  const int h = wave & 1, c0 = (wave >> 1) * 16;
+  constexpr int CSTEP = GCF_WAVES / 2 * 16;
+  auto row_of = [&](int r) { return mod(start + min(row0 + 16 * h + r, n8 - 1) - L / 2); };
+  // this lane's A row of E: root index at a = l4, and its step for a + 4
+  const int u = row_of(l16);
+  const int e0 = mod(u * l4), de = mod(4 * u);
+  for (int b0 = c0; b0 <= R; b0 += CSTEP) {
+    d4 re = {}, im = {};
+    int e = e0;
+    for (int a = l4; a <= R + l4; a += 4) {
+      const double2 x = screen(a, b0 + l16);
+      const double c = coef(a, e);
+      mfma_d(re, c, x.x);
+      mfma_d(im, c, x.y);
+      e += de;
+      e -= e >= L ? L : 0;
     }
+    const double2 x = even ? screen(R, b0 + l16) : make_double2(0.0, 0.0);
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        Y[(16 * h + 4 * i + l4) * yp + b0 + l16] = make_double2(re[h][i], im[h][i]);
+    for (int i = 0; i < 4; i++) {
+      const int r = 4 * i + l4;
+      const double s = root[mod(row_of(r) * R)].y;
+      Y[(16 * h + r) * yp + b0 + l16] = make_double2(fma(s, x.y, re[i]), fma(-s, x.x, im[i]));
+    }
   }
   __syncthreads();
   const double sum = (double)ms * (double)ms;
-  for (int f0 = wave * 16; f0 < n8; f0 += 64) {
+  for (int f0 = c0; f0 < n8; f0 += CSTEP) {
     const int f = min(f0 + l16, n8 - 1);
     const int ov = f / S, sv = f - ov * S;
     const int v = mod(start + 8 * sv + ov - L / 2);
-    int e = mod(v * (l4 - R));
+    int e = mod(v * l4);
     const int d = mod(4 * v);
-    d4 re[2] = {}, im[2] = {};
-    for (int b = l4; b < ms + l4; b += 4) {
-      const double2 x = b < ms ? root[e] : make_double2(0.0, 0.0);
-#pragma unroll
-      for (int h = 0; h < 2; h++) mfma_c(re[h], im[h], Y[(16 * h + l16) * yp + min(b, ms - 1)], x);
+    d4 re = {}, im = {};
+    for (int b = l4; b <= R + l4; b += 4) {
+      const double2 y = Y[(16 * h + l16) * yp + min(b, R)];
+      const double c = coef(b, e);
+      mfma_d(re, y.x, c);
+      mfma_d(im, y.y, c);
       e += d;
       e -= e >= L ? L : 0;
     }
     if (f0 + l16 >= n8) continue;
+    const double s = even ? root[mod(v * R)].y : 0.0;
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int r = row0 + 16 * h + 4 * i + l4;
-        if (r >= n8) continue;
-        T o;
-        o.x = re[h][i] / sum;
-        o.y = im[h][i] / sum;
-        dst[((long long)((r & 7) * GCF_OVER + ov) * S + (r >> 3)) * S + sv] = o;
-      }
+    for (int i = 0; i < 4; i++) {
+      const int r = row0 + 16 * h + 4 * i + l4;
+      if (r >= n8) continue;
+      const double2 y = Y[(16 * h + 4 * i + l4) * yp + R];
+      T o;
+      o.x = fma(s, y.y, re[i]) / sum;
+      o.y = fma(-s, y.x, im[i]) / sum;
+      dst[((long long)((r & 7) * GCF_OVER + ov) * S + (r >> 3)) * S + sv] = o;
+    }
   }
 }
 
@@ -434,7 +446,7 @@ rcg_status launch_layers(const GcfPlanes &pl, int ms, double t2, void *dst, hipS
   const size_t lds = gcf_lds(ms, QUAD);
   RCG_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gcf_layers<T, QUAD>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)GCF_LDS));
-  hipLaunchKernelGGL((k_gcf_layers<T, QUAD>), dim3(pl.first[pl.n]), dim3(256), lds, st, pl, ms, t2,
+  hipLaunchKernelGGL((k_gcf_layers<T, QUAD>), dim3(pl.first[pl.n]), dim3(GCF_THREADS), lds, st, pl, ms, t2,
                      static_cast<T *>(dst));
   RCG_HIP_TRY(hipGetLastError());
   return RCG_OK;
