@@ -499,6 +499,14 @@ rcg_status rcg_hogbom(void *model, void *res, const void *psf, int f64, int siz,
                       void *scratch, void *stream);
 rcg_status rcg_hogbom_iterations(const void *scratch, unsigned *iters,
                                  void *stream);
+/* The same, for a caller that waits for the result: returns when all is done,
+ * with the accepted peaks in *iters (may be null).  Faster where few parts of
+ * the image can hold the peak, which the host finds out as the work goes on;
+ * rcg_hogbom queues everything without waiting (it may be captured in a
+ * graph).  Both give the same bits. */
+rcg_status rcg_hogbom_run(void *model, void *res, const void *psf, int f64, int siz,
+                          int pitch, unsigned niters, double gain, double threshold,
+                          void *scratch, unsigned *iters, void *stream);
 
 #ifdef __cplusplus
 }

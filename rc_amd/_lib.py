@@ -118,6 +118,8 @@ SIGNATURES: dict[str, tuple] = {
     "rcg_hogbom": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, C.c_int, C.c_uint, C.c_double,
                              C.c_double, vp, vp]),
     "rcg_hogbom_iterations": (C.c_int, [vp, C.POINTER(C.c_uint), vp]),
+    "rcg_hogbom_run": (C.c_int, [vp, vp, vp, C.c_int, C.c_int, C.c_int, C.c_uint, C.c_double,
+                                 C.c_double, vp, C.POINTER(C.c_uint), vp]),
     # reference host entry points next to the gridder
     "normalizeCPU": (None, [vp, C.c_int, C.c_int]),
     "rotateCPU": (None, [vp, vp, C.c_int, C.c_double]),

@@ -29,19 +29,33 @@
 //   k_clean_minor   one workgroup, up to CK iterations: 4 tiles per thread in
 //                   registers, candidates visited by quarters, a
 //                   wavefront each;
-// then k_clean_tiles again.  No host synchronisation.
+// then k_clean_tiles again.
+//
+// How many tiles can hold the peak is a matter of the PSF and the image: with
+// the sidelobes of a short snapshot, or on a flat image, the slacks soon let in
+// hundreds, all visited by one CU (100 points on 2048^2: 93 an iteration, 87
+// us; a zero image: all, 6.7 ms).  So k_clean_minor stops before it visits more
+// than a budget (visit_budget, below), and the rest is done by passes over the
+// whole image, one launch per iteration (k_clean_pass: every block reduces the
+// last pass's 512 block maxima, subtracts the component and leaves its own
+// maximum): 12 us an iteration at 2048^2 FP32 whatever the image.  The host has
+// to see that, so rcg_hogbom_run waits for the result; rcg_hogbom, which
+// queues everything at once, is passes only.
 //
 // What bounds it: k_clean_minor the latency of an iteration on one CU (three
 // barriers, one round of loads per visit), k_clean_tiles the reads of the PSF
-// beyond the L2 (16 MB a component at 2048^2 FP32, 10 TB/s).  Measured, 1000
-// FP32 iterations on a 2048^2 dirty image: 10.1 ms against 16.9 ms for one
-// pass over the whole image per iteration (a launch each, every block reducing
-// the last pass's 512 block maxima first); two major cycles of 100 iterations
-// at 1024^2: 2.2 against 4.2 ms.  CK iterations between two rounds of
+// beyond the L2 (16 MB a component at 2048^2 FP32, 10 TB/s), k_clean_pass its
+// launch and the image's and PSF's bytes.  Measured, FP32, an iteration on
+// tiles and by a pass: dense uv coverage 10.0 and 12.7 us at 2048^2, 7.7 and
+// 10.3 at 1024^2; 2000 points 16.9 and 12.3, 10.0 and 10.2; 100 points 87 and
+// 12, 48 and 10.  Passes whose reductions shuffled value, sign and place took
+// 16.9 us at 2048^2, 13 at 256^2 (6.7 now).  CK iterations between two rounds of
 // k_clean_tiles: a tile seldom visited has up to CK components to catch up on,
 // a round costs 10 us besides them; 12 and 24 are within 1% of 16, 32 takes
 // 10.4, 64 11.4, 128 15.3 ms.  A visit's pixels four to a lane, loaded
 // together: 13 us an iteration at CK = 128, against 18 us one to a lane.
+#include <algorithm>
+
 #include "rcg_internal.h"
 
 namespace rcg {
@@ -54,6 +68,8 @@ constexpr int CK = 16;         // iterations (components) between two rounds of 
 constexpr int CAND = 128;      // tiles visited at a time
 constexpr int NP = 4;          // parts of a tile, a wavefront each
 constexpr int MSIDE = 65;      // side of the table of PSF maxima at most
+constexpr int PBLOCKS = 512;   // blocks of a pass over the whole image
+constexpr int PB = 8;          // pixels of a thread whose loads are issued together
 
 struct CleanState {
   long long pos;    // residual peak (row*pitch + col)
@@ -62,6 +78,7 @@ struct CleanState {
   double pval;      // signed PSF peak value
   int done;
   int iters;
+  int passes;       // too many tiles can hold the peak: passes from here on
 };
 
 // A tile's maximum: |value|, the signed value, its place in the tile (row-major).
@@ -75,6 +92,12 @@ struct Comp {
   int dr, dc;  // row and column of the PSF over pixel (0, 0)
 };
 
+// Block maxima of a pass: |value|, signed value, row-major place in the image.
+struct Partials {
+  double a[PBLOCKS], v[PBLOCKS];
+  long long p[PBLOCKS];
+};
+
 struct Scratch {
   CleanState st;
   int nc;                    // pending components
@@ -83,6 +106,7 @@ struct Scratch {
   unsigned char applied[CTILES];  // of the pending, how many a tile has had
   TileMax psf[CTILES], res[CTILES];
   float m2[MSIDE * MSIDE];   // largest |psf| over tiles (i-1, i) x (j-1, j)
+  Partials part[2];          // of the last pass and of the one before it
 };
 
 // Tile geometry: nb x nb tiles of 2^lb pixels a side.
@@ -155,22 +179,45 @@ __device__ __forceinline__ T lanes_max(T x)
   x = dpp_max<0x143>(x);
   return lane_value(x, 63);
 }
-// The largest a (>= 0) of the lanes in `among`, the lowest place p on ties,
-// and its v; a = -1 when there is none.
+// The same for the lowest of whole numbers (a lane without a source keeps its own).
+template <int CTRL>
+__device__ __forceinline__ long long dpp_min(long long w)
+{
+  const int lo = __builtin_amdgcn_update_dpp((int)w, (int)w, CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(w >> 32), (int)(w >> 32), CTRL, 0xf, 0xf, false);
+  const long long x = (long long)hi << 32 | (unsigned)lo;
+  return x < w ? x : w;
+}
+template <bool ROW>
+__device__ __forceinline__ long long lanes_min(long long w)
+{
+  w = dpp_min<0x111>(w);
+  w = dpp_min<0x112>(w);
+  w = dpp_min<0x114>(w);
+  w = dpp_min<0x118>(w);
+  if (ROW) return lane_word(w, 15);
+  w = dpp_min<0x142>(w);
+  w = dpp_min<0x143>(w);
+  return lane_word(w, 63);
+}
+// The largest a (>= 0) of the lanes, the lowest place p on ties, and its v; a
+// = -1 when there is none.  (On a flat image all lanes tie: one by one they
+// took 3 us a reduction.)
 template <bool ROW, class T>
-__device__ __forceinline__ void lanes_best(T &a, T &v, long long &p, unsigned long long among)
+__device__ __forceinline__ void lanes_best(T &a, T &v, long long &p)
 {
   const T m = lanes_max<ROW>(a);
-  unsigned long long eq = m >= 0 ? __ballot(a == m) & among : 0;
-  T bv = 0;
+  unsigned long long eq = m >= 0 ? __ballot(a == m) : 0;
   long long bp = 0x7fffffffffffffffLL;
-  for (; eq; eq &= eq - 1) {
+  T bv = 0;
+  if (eq & (eq - 1)) {
+    bp = lanes_min<ROW>(a == m ? p : bp);
+    eq &= __ballot(p == bp);
+  }
+  if (eq) {
     const int l = __ffsll(eq) - 1;
-    const long long q = lane_word(p, l);
-    if (q < bp) {
-      bp = q;
-      bv = lane_value(v, l);
-    }
+    bp = lane_word(p, l);
+    bv = lane_value(v, l);
   }
   a = m;
   v = bv;
@@ -288,7 +335,7 @@ __device__ __forceinline__ TileMax visit(T *__restrict__ img, const T *__restric
     }
   }
   long long p = bp;
-  lanes_best<false>(ba, bv, p, ~0ull);
+  lanes_best<false>(ba, bv, p);
   return TileMax{(double)ba, (double)bv, ba >= 0 ? (int)p : 0x7fffffff, 0};
 }
 
@@ -327,7 +374,7 @@ struct BlockBest {
 template <class T>
 __device__ __forceinline__ void block_take(T &a, T &v, long long &p, BlockBest<T> &sh)
 {
-  lanes_best<false>(a, v, p, ~0ull);
+  lanes_best<false>(a, v, p);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) {
     sh.a[wave] = a;
@@ -335,10 +382,11 @@ __device__ __forceinline__ void block_take(T &a, T &v, long long &p, BlockBest<T
     sh.p[wave] = p;
   }
   __syncthreads();
-  a = sh.a[lane & 15];
-  v = sh.v[lane & 15];
-  p = sh.p[lane & 15];
-  lanes_best<true>(a, v, p, 0xffffull);
+  const int w = lane & ((blockDim.x >> 6) - 1);  // 8 or 16 wavefronts
+  a = sh.a[w];
+  v = sh.v[w];
+  p = sh.p[w];
+  lanes_best<true>(a, v, p);
 }
 
 constexpr long long NOWHERE = 0x7fffffffffffffffLL;
@@ -366,7 +414,7 @@ k_clean_prep(Tiling g, Scratch *__restrict__ sc)
   if (threadIdx.x == 0) {
     const bool any = p != NOWHERE;
     const int pr = any ? (int)(p / g.siz) : 0, pc = any ? (int)(p % g.siz) : 0;
-    sc->st = CleanState{0, (long long)pr * g.pitch + pc, 0.0, any ? v : 0.0, 0, 0};
+    sc->st = CleanState{0, (long long)pr * g.pitch + pc, 0.0, any ? v : 0.0, 0, 0, 0};
     sc->prow = pr;
     sc->pcol = pc;
     sc->nc = 0;
@@ -387,11 +435,14 @@ k_clean_prep(Tiling g, Scratch *__restrict__ sc)
 }
 
 // Up to `iters` (<= CK) iterations.  Three barriers an iteration: after the
-// candidates' list, the visits, and the new component.
+// candidates' list, the visits, and the new component.  The run ends, and with
+// it the work on tiles, before it visits more than `budget` of them.  The
+// state goes to the host's copy too.
 template <class T>
 __global__ void __launch_bounds__(CT)
 k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ model, Tiling g,
-              Scratch *__restrict__ sc, double gain, double threshold, int iters)
+              Scratch *__restrict__ sc, double gain, double threshold, int iters, int budget,
+              CleanState *__restrict__ seen)
 {
 #pragma clang fp contract(off)
   __shared__ float m2[MSIDE * MSIDE];
@@ -403,7 +454,7 @@ k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ mo
   __shared__ int n_cand[2];  // the round's count; the other is cleared for the next
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (sc->st.done) {
+  if (sc->st.done || sc->st.passes) {
     if (tid == 0) sc->nc = 0;
     return;
   }
@@ -426,7 +477,7 @@ k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ mo
     s[j] = LEAST;
   }
   if (tid < 2) n_cand[tid] = 0;
-  int nc = 0, done = 0, flip = 0;
+  int nc = 0, done = 0, passes = 0, flip = 0, visits = 0;
   long long pos = 0;
   double val = 0.0;
   // A bound from below on the image's maximum: the largest e - s.
@@ -458,6 +509,11 @@ k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ mo
       }
       __syncthreads();
       const int all = __builtin_amdgcn_readfirstlane(n_cand[flip]), n = min(all, CAND);
+      visits += all;
+      if (visits > budget) {
+        passes = 1;
+        break;
+      }
       if (tid == 0) n_cand[flip ^ 1] = 0;
       flip ^= 1;
       for (int job = wave; job < n * NP; job += CT / 64) {
@@ -479,7 +535,7 @@ k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ mo
             p = image_place(g, cand[(k + lane) / NP], m.p);
           }
         }
-        lanes_best<false>(a, v, p, ~0ull);
+        lanes_best<false>(a, v, p);
         take(ba, bv, bp, a, v, p);
       }
 #pragma unroll
@@ -497,6 +553,7 @@ k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ mo
       lb = (float)ba * (1.f - 4.f * TINY);
       __syncthreads();  // the list and the visits have been read
     }
+    if (passes) break;
     if (bp == NOWHERE || fabs((double)bv) < threshold || pval == 0.0) {
       done = 1;
       pos = bp == NOWHERE ? 0 : bp / g.siz * g.pitch + bp % g.siz;
@@ -533,6 +590,114 @@ k_clean_minor(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ mo
     sc->st.val = val;
     sc->st.done = done;
     sc->st.iters = iter0 + nc;
+    sc->st.passes = passes;
+    *seen = sc->st;
+  }
+}
+
+// Pass `it` over the whole image.  it >= 1: reduce the last pass's block maxima
+// (pin) to the peak of iteration base + it - 1; stop below the threshold; else
+// block 0 adds gain * peak / psf peak to the model, and every block subtracts
+// that times the PSF shifted onto the peak.  find: leave this block's maximum
+// of the (updated) image in pout.  it = 0: find only.  The kernel boundary
+// orders the passes: no block waits for another.
+template <class T>
+__global__ void __launch_bounds__(CT)
+k_clean_pass(T *__restrict__ img, const T *__restrict__ psf, T *__restrict__ model, Tiling g,
+             Scratch *__restrict__ sc, double gain, double threshold, int base, int it, int find,
+             const Partials *__restrict__ pin, Partials *__restrict__ pout)
+{
+#pragma clang fp contract(off)
+  __shared__ BlockBest<double> sh_peak, sh_out;
+  CleanState *st = &sc->st;
+  if (st->done) return;
+  const int siz = g.siz, pitch = g.pitch;
+  long long dr = 0, dc = 0;
+  T a = 0;
+  const bool subtract = it > 0;
+  if (subtract) {
+    double pa = -1.0, pv = 0.0;
+    long long pp = NOWHERE;
+    for (int k = threadIdx.x; k < PBLOCKS; k += blockDim.x) take(pa, pv, pp, pin->a[k], pin->v[k], pin->p[k]);
+    block_take(pa, pv, pp, sh_peak);
+    const long long r = pp == NOWHERE ? 0 : pp / siz, c = pp == NOWHERE ? 0 : pp % siz;
+    const long long pos = r * pitch + c;
+    const double pval = st->pval;
+    if (pp == NOWHERE || fabs(pv) < threshold || pval == 0.0) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->pos = pos;
+        st->val = pv;
+        st->done = 1;
+      }
+      return;
+    }
+    const double w = gain * pv / pval;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      st->pos = pos;
+      st->val = pv;
+      st->iters = base + it;
+      model[pos] += (T)w;
+    }
+    dr = sc->prow - r;
+    dc = sc->pcol - c;
+    a = (T)w;
+  }
+  // A thread's pixels are rows blockIdx.x + k * gridDim.x, columns
+  // threadIdx.x + j * blockDim.x, taken PB at a time in (k, j) order.  Every
+  // load of a batch (image, and PSF where the shifted PSF covers the pixel)
+  // is issued before any is used, so a batch costs one memory latency: at
+  // 2048^2 a thread's 8 pixels are one batch.  The pixels of a batch are
+  // distinct and img and psf do not alias, so the stores may follow all the
+  // loads.  The thread's running maximum: its pixels come in increasing
+  // order, so a strict > keeps the first on ties, as take() does.
+  T ba = -1, bv = 0;
+  int br = -1, bc = 0;
+  const int tx = threadIdx.x, bx = blockIdx.x, nb = gridDim.x, nt = blockDim.x;
+  const int nj = tx < siz ? (siz - 1 - tx) / nt + 1 : 0;
+  const int nk = bx < siz ? (siz - 1 - bx) / nb + 1 : 0;
+  const int ne = nj * nk;
+  int k = 0, j = 0;
+  for (int e0 = 0; e0 < ne; e0 += PB) {
+    T x[PB], p[PB];
+    int rr[PB], cc[PB];
+    bool sb[PB];
+#pragma unroll
+    for (int u = 0; u < PB; u++) {
+      const int r = bx + k * nb, c = tx + j * nt;
+      const bool ok = e0 + u < ne;
+      const long long sr = r + dr, sc = c + dc;
+      rr[u] = r;
+      cc[u] = c;
+      sb[u] = ok && subtract && sr >= 0 && sr < siz && sc >= 0 && sc < siz;
+      x[u] = ok ? img[(long long)r * pitch + c] : T(0);
+      p[u] = sb[u] ? psf[sr * pitch + sc] : T(0);
+      if (++j == nj) {
+        j = 0;
+        k++;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PB; u++) {
+      if (sb[u]) {
+        x[u] -= a * p[u];
+        img[(long long)rr[u] * pitch + cc[u]] = x[u];
+      }
+      if (find && e0 + u < ne && fabs(x[u]) > ba) {
+        ba = fabs(x[u]);
+        bv = x[u];
+        br = rr[u];
+        bc = cc[u];
+      }
+    }
+  }
+  if (!find) return;
+  double ma = br >= 0 ? (double)ba : -1.0, mv = (double)bv;
+  long long mp = br >= 0 ? (long long)br * siz + bc : NOWHERE;
+  block_take(ma, mv, mp, sh_out);
+  if (tx == 0) {
+    pout->a[blockIdx.x] = ma;
+    pout->v[blockIdx.x] = mv;
+    pout->p[blockIdx.x] = mp;
   }
 }
 
@@ -544,26 +709,138 @@ __global__ void k_zero(T *__restrict__ p, long long n)
     p[i] = 0;
 }
 
+// The model cleared, the PSF's peak and maxima, the state.
+template <class T>
+void begin(T *model, const T *psf, const Tiling &g, Scratch *sc, hipStream_t st)
+{
+  hipLaunchKernelGGL(k_zero<T>, dim3(1024), dim3(256), 0, st, model, (long long)g.siz * g.pitch);
+  hipLaunchKernelGGL(k_clean_tiles<T>, dim3(g.nb * g.nb), dim3(256), 0, st, const_cast<T *>(psf),
+                     psf, g, sc, 1, 0);
+  hipLaunchKernelGGL(k_clean_prep, dim3(1), dim3(CT), 0, st, g, sc);
+}
+
+// Iterations [base, niters), one launch each after the first that finds the
+// peak only.
+template <class T>
+void passes(T *model, T *res, const T *psf, const Tiling &g, unsigned base, unsigned niters,
+            double gain, double threshold, Scratch *sc, hipStream_t st)
+{
+  // FP64 passes need more registers per thread: 512 threads keep two blocks
+  // per CU resident
+  const int nt = sizeof(T) == 8 ? 512 : CT;
+  Partials *pp = sc->part;
+  const unsigned n = niters - base;
+  for (unsigned it = 0; n && it <= n; it++)
+    hipLaunchKernelGGL(k_clean_pass<T>, dim3(PBLOCKS), dim3(nt), 0, st, res, psf, model, g, sc, gain,
+                       threshold, (int)base, (int)it, it < n ? 1 : 0, pp + ((it + 1) & 1),
+                       pp + (it & 1));
+}
+
 template <class T>
 rcg_status hogbom(T *model, T *res, const T *psf, int siz, int pitch, unsigned niters,
-                  double gain, double threshold, void *scratch, hipStream_t st)
+                  double gain, double threshold, Scratch *sc, hipStream_t st)
 {
-  Scratch *sc = static_cast<Scratch *>(scratch);
   const Tiling g = tiling_of(siz, pitch);
-  const int nt = g.nb * g.nb;
-  hipLaunchKernelGGL(k_zero<T>, dim3(1024), dim3(256), 0, st, model, (long long)siz * pitch);
-  hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, const_cast<T *>(psf), psf, g,
-                     sc, 1, 0);
-  hipLaunchKernelGGL(k_clean_prep, dim3(1), dim3(CT), 0, st, g, sc);
-  if (niters > 0)
-    hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, res, psf, g, sc, 0, 0);
-  for (unsigned done = 0; done < niters; done += CK) {
-    const int n = (int)(niters - done < (unsigned)CK ? niters - done : (unsigned)CK);
-    hipLaunchKernelGGL(k_clean_minor<T>, dim3(1), dim3(CT), 0, st, res, psf, model, g, sc, gain,
-                       threshold, n);
-    hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, res, psf, g, sc, 0, 1);
-  }
+  begin(model, psf, g, sc, st);
+  passes(model, res, psf, g, 0, niters, gain, threshold, sc, st);
   RCG_HIP_TRY(hipGetLastError());
+  return RCG_OK;
+}
+
+// Tiles a run of CK iterations may visit before passes are the faster way (0:
+// from the start).  A pass takes 6.5 us and 0.37 us a MB of the image; an
+// iteration on tiles about half of that a MB, 5 to 13 us by the tiles' side,
+// and for each visit 0.85, 3 and 14 us with tiles of 32, 64 and 128 pixels.
+// They break even at a number of visits an iteration that grows as the image's
+// bytes over a tile's pixels, as the number of tiles times a pixel's bytes:
+// measured 3.8 and 9.5 at 4096^2 (FP32, FP64; 4.7 and 9.4 by the rule), 2.7 and
+// 5.3 at 3000^2 (2.6, 5.2), 5 and 11 at 8192^2 (4.7, 9.4), 9.5 at 2048^2 FP64.
+// Tiles of 32 pixels, where both sides are bound by latency, break even at 4.2
+// to 6.4 from 400^2 to 2048^2 (5).  Four tiles are always faster than passes
+// (5.6 against 6.9 us at 64^2), from there to 400^2 a pass is (6.8 against 8.7
+// us at 256^2), and below two visits an iteration nothing is left.
+int visit_budget(const Tiling &g, size_t elem)
+{
+  if (g.nb <= 2) return 1 << 30;
+  if (g.siz < 400) return 0;
+  const int rule = (int)(g.nb * g.nb * elem / 218);
+  if (g.lb == 5) return std::max(rule, 5 * CK);
+  return rule < 2 * CK ? 0 : rule;
+}
+
+// What the host keeps of a running call: given back when the stream is done.
+struct Watch {
+  hipStream_t st;
+  CleanState *seen = nullptr;  // pinned host memory
+  hipEvent_t ev[2] = {};
+  ~Watch()
+  {
+    (void)hipStreamSynchronize(st);
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (seen) pool_pin_put(seen);
+  }
+};
+
+// On tiles while that pays, then by passes.  Rounds are queued in groups, each
+// up to twice as large as the last, and before the next group the host looks
+// at where the group before this one has got: the device never waits for it.
+template <class T>
+rcg_status hogbom_run(T *model, T *res, const T *psf, int siz, int pitch, unsigned niters,
+                      double gain, double threshold, Scratch *sc, unsigned *iters, hipStream_t st)
+{
+  const Tiling g = tiling_of(siz, pitch);
+  const int nt = g.nb * g.nb, budget = visit_budget(g, sizeof(T));
+  Watch w{st};
+  RCG_HIP_TRY(pool_pin(reinterpret_cast<void **>(&w.seen)));
+  for (hipEvent_t &e : w.ev) RCG_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  volatile CleanState *seen = w.seen;
+  seen->done = seen->passes = 0;
+  begin(model, psf, g, sc, st);
+  if (!budget) {
+    passes(model, res, psf, g, 0, niters, gain, threshold, sc, st);
+  } else if (niters > 0) {
+    hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, res, psf, g, sc, 0, 0);
+  }
+  unsigned queued = 0, group = 1;
+  for (int k = 0; budget && queued < niters; k++) {
+    for (unsigned r = 0; r < group && queued < niters; r++) {
+      const unsigned n = std::min(niters - queued, (unsigned)CK);
+      hipLaunchKernelGGL(k_clean_minor<T>, dim3(1), dim3(CT), 0, st, res, psf, model, g, sc, gain,
+                         threshold, (int)n, budget, w.seen);
+      hipLaunchKernelGGL(k_clean_tiles<T>, dim3(nt), dim3(256), 0, st, res, psf, g, sc, 0, 1);
+      queued += n;
+    }
+    RCG_HIP_TRY(hipGetLastError());
+    RCG_HIP_TRY(hipEventRecord(w.ev[k & 1], st));
+    if (k > 0) {
+      RCG_HIP_TRY(hipEventSynchronize(w.ev[(k - 1) & 1]));
+      if (seen->done || seen->passes) break;
+    }
+    group = std::min(2 * group, 32u);
+  }
+  auto state = [&]() {
+    hipError_t e = hipMemcpyAsync(w.seen, &sc->st, sizeof(CleanState), hipMemcpyDeviceToHost, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+  };
+  RCG_HIP_TRY(state());
+  if (seen->passes && !seen->done) {
+    passes(model, res, psf, g, (unsigned)seen->iters, niters, gain, threshold, sc, st);
+    RCG_HIP_TRY(hipGetLastError());
+    RCG_HIP_TRY(state());
+  }
+  *iters = (unsigned)seen->iters;
+  return RCG_OK;
+}
+
+rcg_status check_hogbom(const void *model, const void *res, const void *psf, int siz, int pitch,
+                        const void *scratch)
+{
+  if (!model || !res || !psf || !scratch || siz <= 0 || pitch < siz ||
+      (long long)siz * siz > 0x7fffffffffffLL) {
+    set_error(RCG_ERR_ARG, "rcg_hogbom: bad arguments");
+    return RCG_ERR_ARG;
+  }
   return RCG_OK;
 }
 
@@ -582,19 +859,37 @@ extern "C" rcg_status rcg_hogbom(void *model, void *res, const void *psf, int f6
                                  void *scratch, void *stream)
 {
   clear_error();
-  if (!model || !res || !psf || !scratch || siz <= 0 || pitch < siz ||
-      (long long)siz * siz > 0x7fffffffffffLL) {
-    set_error(RCG_ERR_ARG, "rcg_hogbom: bad arguments");
-    return RCG_ERR_ARG;
-  }
+  const rcg_status s = check_hogbom(model, res, psf, siz, pitch, scratch);
+  if (s != RCG_OK) return s;
   hipStream_t st = (hipStream_t)stream;
+  Scratch *sc = static_cast<Scratch *>(scratch);
   if (f64)
     return hogbom<double>(static_cast<double *>(model), static_cast<double *>(res),
                           static_cast<const double *>(psf), siz, pitch, niters, gain,
-                          threshold, scratch, st);
+                          threshold, sc, st);
   return hogbom<float>(static_cast<float *>(model), static_cast<float *>(res),
-                       static_cast<const float *>(psf), siz, pitch, niters, gain, threshold,
-                       scratch, st);
+                       static_cast<const float *>(psf), siz, pitch, niters, gain, threshold, sc,
+                       st);
+}
+
+extern "C" rcg_status rcg_hogbom_run(void *model, void *res, const void *psf, int f64, int siz,
+                                     int pitch, unsigned niters, double gain, double threshold,
+                                     void *scratch, unsigned *iters, void *stream)
+{
+  clear_error();
+  const rcg_status s = check_hogbom(model, res, psf, siz, pitch, scratch);
+  if (s != RCG_OK) return s;
+  unsigned n = 0;
+  if (!iters) iters = &n;
+  hipStream_t st = (hipStream_t)stream;
+  Scratch *sc = static_cast<Scratch *>(scratch);
+  if (f64)
+    return hogbom_run<double>(static_cast<double *>(model), static_cast<double *>(res),
+                              static_cast<const double *>(psf), siz, pitch, niters, gain,
+                              threshold, sc, iters, st);
+  return hogbom_run<float>(static_cast<float *>(model), static_cast<float *>(res),
+                           static_cast<const float *>(psf), siz, pitch, niters, gain, threshold,
+                           sc, iters, st);
 }
 
 // Iterations the last rcg_hogbom on this scratch performed (synchronises).
@@ -632,7 +927,8 @@ extern "C" void deconvolve(double *mod_p, double *res_p, double *psf_p, int siz,
   } else if (hipMemcpyAsync(dr, res_p, bytes, hipMemcpyHostToDevice, st) != hipSuccess ||
              hipMemcpyAsync(dp, psf_p, bytes, hipMemcpyHostToDevice, st) != hipSuccess) {
     set_error(RCG_ERR_HIP, "deconvolve: copy in");
-  } else if (rcg_hogbom(dm, dr, dp, 1, siz, pitch, niters, gain, threshold, ds, st) == RCG_OK) {
+  } else if (rcg_hogbom_run(dm, dr, dp, 1, siz, pitch, niters, gain, threshold, ds, nullptr, st) ==
+             RCG_OK) {
     if (hipMemcpyAsync(mod_p, dm, bytes, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipMemcpyAsync(res_p, dr, bytes, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)

@@ -53,6 +53,10 @@ void pool_put(void *p);
 hipError_t pool_stream(hipStream_t *st);
 void pool_stream_put(hipStream_t st);
 void pool_trim();
+// A pinned host buffer of PIN_BYTES, on the same terms.
+constexpr size_t PIN_BYTES = (size_t)4 << 20;
+hipError_t pool_pin(void **p);
+void pool_pin_put(void *p);
 // A copy between the caller's host memory and the device, after what st holds;
 // done on return, but a small one to the device may still be queued on st.
 hipError_t pool_copy(void *dst, const void *src, size_t bytes, bool to_device, hipStream_t st);

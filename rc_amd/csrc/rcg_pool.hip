@@ -28,7 +28,6 @@ namespace {
 
 constexpr size_t POOL_BYTES = (size_t)4 << 30;
 constexpr size_t POOL_STREAMS = 16;
-constexpr size_t PIN_BYTES = (size_t)4 << 20;  // one staging buffer
 constexpr size_t POOL_PINS = 16;               // kept
 // Copies through staging buffers, by up to COPY_THREADS threads.  Pageable
 // memory moves at 30 GB/s to the device and 17 GB/s back, one thread copying
@@ -204,9 +203,7 @@ void pool_trim()
   p.pins.clear();
 }
 
-namespace {
-
-hipError_t pin_get(void **out)
+hipError_t pool_pin(void **out)
 {
   Pool &p = pool();
   {
@@ -220,7 +217,7 @@ hipError_t pin_get(void **out)
   return hipHostMalloc(out, PIN_BYTES, hipHostMallocDefault);
 }
 
-void pin_put(void *b)
+void pool_pin_put(void *b)
 {
   Pool &p = pool();
   {
@@ -236,13 +233,15 @@ void pin_put(void *b)
   (void)hipHostFree(b);
 }
 
+namespace {
+
 // One thread's share: every chunk it draws, through its own buffer and stream.
 hipError_t copy_chunks(char *dst, const char *src, size_t bytes, size_t chunk, bool to_device,
                        std::atomic<size_t> &next)
 {
   void *pin = nullptr;
   hipStream_t st = nullptr;
-  hipError_t e = pin_get(&pin);
+  hipError_t e = pool_pin(&pin);
   if (e != hipSuccess) return e;
   e = pool_stream(&st);
   while (e == hipSuccess) {
@@ -259,7 +258,7 @@ hipError_t copy_chunks(char *dst, const char *src, size_t bytes, size_t chunk, b
     if (e == hipSuccess && !to_device) memcpy(dst + at, pin, n);
   }
   if (st) pool_stream_put(st);
-  pin_put(pin);
+  pool_pin_put(pin);
   return e;
 }
 

@@ -401,13 +401,11 @@ def hogbom(res: torch.Tensor, psf: torch.Tensor, niters: int, gain: float, thres
     h = _lib.lib()
     scratch = torch.empty(int(h.rcg_hogbom_scratch_bytes()), dtype=torch.uint8,
                           device=res.device)
-    s = _stream(stream)
-    _lib.check(h.rcg_hogbom(model.data_ptr(), res.data_ptr(), psf.data_ptr(),
-                            int(res.dtype == torch.float64), siz, pitch, niters, gain,
-                            threshold, scratch.data_ptr(), s), "rcg_hogbom")
     it = C.c_uint()
-    _lib.check(h.rcg_hogbom_iterations(scratch.data_ptr(), C.byref(it), s),
-               "rcg_hogbom_iterations")
+    _lib.check(h.rcg_hogbom_run(model.data_ptr(), res.data_ptr(), psf.data_ptr(),
+                                int(res.dtype == torch.float64), siz, pitch, niters, gain,
+                                threshold, scratch.data_ptr(), C.byref(it), _stream(stream)),
+               "rcg_hogbom_run")
     return model, int(it.value)
 
 
