@@ -135,6 +135,7 @@ int hipEventCreate(void **e)
   *e = malloc(1);
   return OK;
 }
+int hipEventCreateWithFlags(void **e, unsigned) { return hipEventCreate(e); }
 int hipEventDestroy(void *e)
 {
   free(e);
