@@ -3,7 +3,7 @@
 // One launch covers every point.  Gridding: one wavefront handles one point at
 // a time, its lanes cover the point's S x S window (rows of min(S,64) lanes)
 // and add every tap to HBM with a native FP64 atomic (global_atomic_add_f64).
-// Degridding: 16 lanes a point, summed across them with shuffles.  Arithmetic follows the reference's
+// Degridding: 16 or 64 lanes a point, summed across them with shuffles.  Arithmetic follows the reference's
 // complex product (scatter_gridder_w_dependent_dyn_1p.cpp:169 grid,
 // :171 degrid) in FP64 with contraction switched off.  This is the
 // straightforward GPU gridder and the denominator the tiled FP32 path is
@@ -56,14 +56,19 @@ k_grid_plain_f64(const rcg_pg *__restrict__ pg,
   }
 }
 
-// 16 lanes per point, four points per wavefront: a point's lanes take the taps
-// of its window in row order, 16 apart, four steps' loads together.  Bound by
-// the latency of a point's chain (record, taps and cells, sums, store), which
-// four points now share: 500,310 points of supports 8..24 on 1024^2 0.092
-// against 0.167 ms with a wavefront per point, 2,496,960 of 8..48 on 2048^2
-// 0.41 against 0.81 ms.
-constexpr int PL = 16;
-
+// PL lanes per point: they take the taps of its window in row order, PL apart,
+// U steps' loads together.  Of many points, 16 lanes each: four share a
+// wavefront and the latency of its chain (record, taps and cells, sums,
+// store): 500,310 points of supports 8..24 on 1024^2 0.092 against 0.167 ms
+// with a wavefront per point, 2,496,960 of 8..48 on 2048^2 0.41 against 0.81.
+// Of few, up to FEW_POINTS, a wavefront each: there are lanes enough, and the
+// S^2 / 16 steps of a large window would be the time (100 points of 64 x 64:
+// 11 against 33 us, 1000 of 128 x 128: 89 against 149, 4096: 125 against 155;
+// 8000 of 32, 64, 128: 24, 81, 349 against 21, 65, 229).  More of their steps
+// together help only where the caches do not bound (3000 of 256 x 256: 366 us
+// with one, 433 with two, 514 with four).  (The sums' order, by lane, differs;
+// all of it is FP64.)
+template <int PL, int U>
 __global__ void __launch_bounds__(256)
 k_degrid_plain_f64(const rcg_pg *__restrict__ pg,
                    const double2 *__restrict__ grid,
@@ -94,10 +99,10 @@ k_degrid_plain_f64(const rcg_pg *__restrict__ pg,
       const double2 *t = taps + r.tap0 + (long long)row * st + col;
       const double2 *g = grid + r.cell + (long long)row * pitch + col;
       const long long dt = (long long)dr * st + dc, dg = (long long)dr * pitch + dc;
-      for (int q = sub; q < total; q += 4 * PL) {
-        double2 tt[4], gg[4];
+      for (int q = sub; q < total; q += U * PL) {
+        double2 tt[U], gg[U];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
+        for (int u = 0; u < U; u++) {
           const bool act = q + u * PL < total;
           tt[u] = act ? *t : make_double2(0.0, 0.0);
           gg[u] = act ? *g : make_double2(0.0, 0.0);
@@ -111,7 +116,7 @@ k_degrid_plain_f64(const rcg_pg *__restrict__ pg,
           }
         }
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
+        for (int u = 0; u < U; u++) {
           const double ty = tt[u].y * sgn;
           const double pr = gg[u].x * tt[u].x - gg[u].y * ty;
           const double pi = gg[u].x * ty + gg[u].y * tt[u].x;
@@ -135,6 +140,8 @@ __global__ void k_zero_f64(double *__restrict__ p, long long n)
        i += (long long)gridDim.x * blockDim.x)
     p[i] = 0.0;
 }
+
+constexpr long long FEW_POINTS = 6144;
 
 static int plain_blocks(long long n)
 {
@@ -192,9 +199,10 @@ extern "C" rcg_status rcg_degrid_plain_f64(const rcg_geom *geom,
   if (s != RCG_OK) return s;
   const long long n = (long long)geom->n_chunks * geom->ts_ch;
   if (n == 0) return RCG_OK;
-  hipLaunchKernelGGL(k_degrid_plain_f64, dim3(plain_blocks((n + 3) / 4)), dim3(256), 0,
-                     (hipStream_t)stream, pg,
-                     reinterpret_cast<const double2 *>(grid),
+  const bool few = n <= FEW_POINTS;
+  hipLaunchKernelGGL(few ? (k_degrid_plain_f64<64, 1>) : (k_degrid_plain_f64<16, 4>),
+                     dim3(plain_blocks(few ? n : (n + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+                     pg, reinterpret_cast<const double2 *>(grid),
                      reinterpret_cast<const double2 *>(gcf->data),
                      reinterpret_cast<double2 *>(vis), geom->grid_pitch, n);
   RCG_HIP_TRY(hipGetLastError());
