@@ -838,6 +838,12 @@ hipError_t blocks_of(int *gb, int *db)
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &dg, reinterpret_cast<const void *>(&k_degrid_halo<T, H>), 64, 0);
   if (e != hipSuccess) return e;
+  // A gridding workgroup is one wavefront: whole fours of them a CU, so that
+  // its four SIMDs hold the same number.  With the five that the LDS lets in
+  // (32 KB regions) two share a SIMD, and every workgroup has an item from
+  // the start: 100,000 points of 64 x 64 (1216 items) 535 us against 365,
+  // 400,000 of 48 x 48 (1805) 1412 against 1150.
+  if (g > 4) g &= ~3;
   // a multiple of 8: one share per XCD
   *gb = std::max(8, (std::max(1, g) * std::max(1, cus)) & ~7);
   *db = std::max(8, (std::max(1, dg) * std::max(1, cus)) & ~7);

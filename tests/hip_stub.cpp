@@ -21,6 +21,8 @@ constexpr int OK = 0, NOMEM = 2;
 std::mutex mu;
 size_t live = 0, limit = (size_t)1 << 30, n_free = 0;
 std::atomic<long> launches{0};
+int per_cu = 2;                 // workgroups of a kernel on a CU
+unsigned last_grid[1025] = {};  // blocks of the last launch, by threads a block
 thread_local int last_error = OK;
 thread_local int fail_new = 0;  // the fail_new-th operator new from here on throws
 thread_local Dim3 cfg_grid, cfg_block;
@@ -48,6 +50,8 @@ void stub_limit(size_t bytes) { limit = bytes; }
 size_t stub_live() { return live; }
 size_t stub_frees() { return n_free; }
 long stub_launches() { return launches; }
+void stub_per_cu(int n) { per_cu = n; }
+unsigned stub_last_grid(int threads) { return last_grid[threads]; }
 void stub_fail_new(int n) { fail_new = n; }
 int stub_new_left() { return fail_new; }
 
@@ -115,7 +119,7 @@ int hipDeviceGetAttribute(int *v, int, int)
 }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t)
 {
-  *n = 2;
+  *n = per_cu;
   return OK;
 }
 int hipFuncSetAttribute(const void *, int, int) { return OK; }
@@ -159,9 +163,10 @@ int __hipPopCallConfiguration(Dim3 *g, Dim3 *b, size_t *lds, void **st)
   *st = cfg_stream;
   return OK;
 }
-int hipLaunchKernel(const void *, Dim3, Dim3, void **, size_t, void *)
+int hipLaunchKernel(const void *, Dim3 grid, Dim3 block, void **, size_t, void *)
 {
   launches++;
+  if (block.x <= 1024) last_grid[block.x] = grid.x;
   return OK;
 }
 int hipGetLastError()
