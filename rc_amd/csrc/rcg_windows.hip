@@ -88,7 +88,11 @@ struct Walk {
   int k, n;               // step and steps of this lane
 };
 
-// The next U steps; past its last a lane reads zeros.
+// The next U steps; past its last a lane reads zeros.  The second half of an
+// odd row's last load lies past the row, and of the table's very last row past
+// the buffer's end: each dword is checked against the end by itself, so that
+// the tap in the first half is read (observed for loads 1 to 4 dwords before
+// the end; the last tap of a table is tested).
 template <bool ODD>
 __device__ __forceinline__ void win_load(Steps &s, Walk &w, int dummy, __amdgpu_buffer_rsrc_t rsrc)
 {
