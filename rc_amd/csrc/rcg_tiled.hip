@@ -911,7 +911,7 @@ k_degrid_tiles_f64(TiledDev d, const double2 *__restrict__ grid,
     }
     __syncthreads();
     for (int k = ir.begin + wave; k < ir.end; k += F64_WAVES) {
-      const int4 rec = d.pairs[k];
+      const int4 rec = uniform_record(d.pairs, k);
       const int r0 = rec.x & 63, c0 = (rec.x >> 6) & 63;
       const int w = ((rec.x >> 12) & 63) + 1;
       const int rows = ((rec.x >> 18) & 63) + 1;

@@ -37,6 +37,18 @@ struct ItemRange {
   long long goff;          // element offset of the instance's grid
 };
 
+// Record k of a plan, the same k in all lanes, by the scalar path: binning is
+// an earlier kernel, so the records are constant here, which the compiler
+// cannot see past the work queue's atomics (it loads them per lane: 8% of
+// k_degrid_tiles_f64's time).
+__device__ __forceinline__ int4 uniform_record(const int4 *p, int k)
+{
+  typedef int Word4 __attribute__((ext_vector_type(4)));
+  typedef const __attribute__((address_space(4))) Word4 *ConstPtr;
+  const Word4 r = *(ConstPtr)(unsigned long long)(p + __builtin_amdgcn_readfirstlane(k));
+  return make_int4(r[0], r[1], r[2], r[3]);
+}
+
 __device__ __forceinline__ ItemRange item_of(const TiledDev &d, int item)
 {
   const int4 it = d.items[item];
