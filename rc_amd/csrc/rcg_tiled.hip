@@ -734,7 +734,10 @@ k_grid_tiles(TiledDev d, const float2 *__restrict__ vis,
 // in FP64 without contraction, the same value the plain FP64 gridder adds;
 // only the order of the sums differs.  The workgroup's wavefronts share one
 // FP64 copy of the tile and add into it with LDS FP64 atomics (ds_add_f64):
-// at T = 32 a copy is 17 KB, so nine workgroups fit a CU.  Real and imaginary
+// at T = 32 a copy is 17 KB, so eight workgroups, all the wavefronts a CU
+// takes, fit one; without the bound below 112 SGPRs left room for seven, and
+// 2038 items of 100 x 100 windows made a second round (1118 against 809 us).
+// Real and imaginary
 // parts lie in planes of their own: 64 lanes on consecutive cells take 9
 // cycles an atomic there and 17 interleaved.  Records come 64 at a time and
 // the next pair's first taps fly while a pair is added; a pair is tested
@@ -750,7 +753,7 @@ k_grid_tiles(TiledDev d, const float2 *__restrict__ vis,
 constexpr int F64_WAVES = 4;  // 2: 3.7 ms, 8: 3.2-3.5 ms on the workload above
 
 template <int T>
-__global__ void __launch_bounds__(64 * F64_WAVES)
+__global__ void __launch_bounds__(64 * F64_WAVES, T == 64 ? 2 : 8)  // wavefronts per SIMD
 k_grid_tiles_f64(TiledDev d, const double2 *__restrict__ vis,
                  const double2 *__restrict__ taps, long long n_taps,
                  double2 *__restrict__ grid, int add)

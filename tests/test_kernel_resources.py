@@ -34,6 +34,15 @@ def kernels(code):
     return out
 
 
+@pytest.mark.parametrize("tile", [16, 32])
+@pytest.mark.parametrize("kernel", ["k_grid_tiles_f64", "k_degrid_tiles_f64"])
+def test_eight_workgroups_a_cu(code, kernel, tile):
+    """Eight workgroups of four wavefronts: at most 64 VGPRs and 96 SGPRs (an
+    allocation of 112 leaves room for seven)."""
+    (sgpr, vgpr), = [v for n, v in kernels(code).items() if f"{kernel}ILi{tile}E" in n]
+    assert sgpr <= 96 and vgpr <= 64
+
+
 @pytest.mark.parametrize("tile", [16, 32, 64])
 def test_records_by_the_scalar_path(code, tile):
     """The FP64 degridder's vector loads are the item's range (two or three),
