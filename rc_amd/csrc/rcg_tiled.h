@@ -55,7 +55,8 @@ struct TiledDev {
   int *tile_start;   // first pair of each tile
   int *tile_cursor;  // fill cursors
   int *item_start;   // first work item of each tile
-  int4 *items;       // work items: first pair, end, tile, 1 if the tile's only one
+  int4 *items;       // work items: first pair, end, tile, pairs of the tile's fullest
+                     // item (bit 31: it is the tile's only one)
   int *totals;       // [0] pairs, [1] items, [3] points above d.windows
   int *seg;          // scan scratch: 2 ints per segment of 1024 tiles
   int *queue;        // N_QUEUE work counters
@@ -109,9 +110,9 @@ rcg_status halo_degrid(const TiledDev &d, int blocks, const float2 *grid, const 
 rcg_status halo_sort_items(const TiledDev &d, hipStream_t st);
 
 // FP32 degridding of whole windows (rcg_windows.hip): whether a plan's tile
-// and supports fit its LDS, its persistent workgroups for `waves` (2, 4 or 8)
-// wavefronts each, and its launch.
-bool windows_fit(int T, int max_support);
+// and supports fit its LDS and its items hold points enough, its persistent
+// workgroups for `waves` (2, 4 or 8) wavefronts each, and its launch.
+bool windows_fit(int T, int max_support, int chunk);
 hipError_t windows_blocks(int T, int max_support, int waves, int *blocks);
 rcg_status windows_degrid(const TiledDev &d, int max_support, int waves, int blocks,
                           const rcg_pg *pg, const float2 *grid, const float2 *taps,

@@ -339,7 +339,7 @@ __device__ __forceinline__ void write_items(const TiledDev &d, int t, int c, int
   auto put = [&](int tile, int cnt, int first, int i, int k) {
     if (i + k < d.item_cap)
       d.items[i + k] = make_int4(first + k * d.chunk, first + min(cnt, (k + 1) * d.chunk), tile,
-                                 cnt <= d.chunk);
+                                 min(cnt, d.chunk) | (cnt <= d.chunk ? 1 << 31 : 0));
   };
   if (m <= 4)
     for (int k = 0; k < m; k++) put(t, c, p0, i0, k);
@@ -1413,7 +1413,7 @@ rcg_status create_plan(const rcg_geom *geoms, int n_inst, int tile, int chunk, i
         break;
     }
   }
-  pl->windows = !halo && windows_fit(tile, max_support);
+  pl->windows = !halo && windows_fit(tile, max_support, chunk);
   d.windows = pl->windows ? max_support : 0;
   if (e == hipSuccess && pl->windows) {
     pl->degrid_waves = WINDOW_WAVES;

@@ -33,6 +33,7 @@ __device__ __forceinline__ void point_tiles(const rcg_pg &r, int pitch, double i
 struct ItemRange {
   int item;                // index of the work item
   int begin, end, single;  // pairs [begin, end); the tile has one item
+  int most;                // pairs of the tile's fullest item
   int tu0, tv0;            // first grid row and column of the tile
   long long goff;          // element offset of the instance's grid
 };
@@ -58,7 +59,8 @@ __device__ __forceinline__ ItemRange item_of(const TiledDev &d, int item)
   ir.item = item;
   ir.begin = it.x;
   ir.end = it.y;
-  ir.single = it.w;
+  ir.single = it.w < 0;
+  ir.most = it.w & 0x7fffffff;
   ir.tu0 = (lt / d.ntx) * d.T;
   ir.tv0 = (lt % d.ntx) * d.T;
   ir.goff = (long long)inst * d.gstride;
@@ -128,7 +130,7 @@ struct ItemQueue {
 };
 
 // Work loop of a persistent workgroup: fn(item range) for every item it
-// draws.  The trailing barrier keeps the next item's LDS writes behind every
+// draws; fn holds a barrier (a wavefront may read the draw late).  The trailing barrier keeps the next item's LDS writes behind every
 // wavefront's use of the current one.  The next draw waits for the end of an
 // item's work: made before it, it hides a latency of 1-2 us, but each
 // workgroup then holds an item in reserve while others run out (4096^2

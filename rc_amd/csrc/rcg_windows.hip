@@ -46,6 +46,20 @@ constexpr int WIN_LDS = 80 * 1024; // two workgroups per CU
 constexpr int U = 4;               // steps whose loads are issued together
 constexpr int G = 8;               // lanes per point
 constexpr int PW = 64 / G;         // points a wavefront takes at a time
+// Points a full item holds (chunk over the tiles that a window meets) from
+// which whole windows are taken: with fewer, most of the 64 points that a
+// workgroup's wavefronts walk at a time are missing, and the region is staged
+// for little.  400,000 points on 2048^2, tile 32, pairs against windows: 31 x 31
+// windows with 17, 34, 51 points an item 330 / 555, 307 / 333, 305 / 266 us, 63
+// x 63 with 15, 30, 59 902 / 1815, 891 / 1003, 912 / 678; 60,000 on 1024^2 with
+// 17, 26 and 7, 30, 45: 98 / 95, 93 / 70 and 189 / 512, 183 / 192, 195 / 160.
+constexpr int ITEM_POINTS = 30;
+// Points of a tile's item up to which each takes a wavefront and reads the grid
+// where it lies.  Uniform points on 4096^2, 16 x 16 and 63 x 63 windows, 0.3
+// points a tile: 89 -> 40 and 456 -> 124 us; 3.7: 187 -> 106 and 1017 -> 450.
+// With up to 4 alike, but 670 us for the last; with up to 16, tiles that hold
+// so many lose (5000 points of 48 x 48 on 512^2, 20 a tile: 22 -> 38 us).
+constexpr int FEW = 6;
 
 // Side of the staged region and its row stride (odd, so that rows start in
 // different banks).
@@ -265,10 +279,60 @@ __device__ __forceinline__ void win_stream(const int4 *pts, int total, int wave,
   } while (left);
 }
 
+// One point by a wavefront, the grid read where it lies: g0 its first cell, tap0
+// its first tap (element).  Lanes take the taps of the window in row order, 64
+// apart, U steps' loads together; sums as in win_add.
+__device__ __forceinline__ float2 win_point(const float2 *__restrict__ g0, int pitch,
+                                            __amdgpu_buffer_rsrc_t rsrc, int tap0, int stride,
+                                            int S, bool conj, int lane)
+{
+  // quotients by the approximate reciprocal: (x + 0.5) / S lies at least 0.5 /
+  // S >= 1/512 from an integer, far above its error
+  const float inv = __builtin_amdgcn_rcpf((float)S);
+  const int row = (int)(((float)lane + 0.5f) * inv), dr = (int)(64.5f * inv);
+  const int dc = 64 - dr * S, total = S * S;
+  int col = lane - row * S;
+  int t = tap0 + row * stride + col, g = row * pitch + col;
+  const int dt = dr * stride + dc, dg = dr * pitch + dc;
+  Acc acc = {};
+  for (int q = lane; q < total + lane; q += 64 * U) {
+    float2 tt[U], gg[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool act = q + 64 * u < total;
+      tt[u] = tap_load(rsrc, act ? (unsigned)t * 8u : TAP_OOB, 0);
+      gg[u] = act ? g0[g] : make_float2(0.f, 0.f);
+      const bool wrap = col + dc >= S;
+      col += wrap ? dc - S : dc;
+      t += wrap ? dt + stride - S : dt;
+      g += wrap ? dg + pitch - S : dg;
+    }
+    float P = 0.f, Q = 0.f, R = 0.f, V = 0.f;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      P = fmaf(gg[u].x, tt[u].x, P);
+      Q = fmaf(gg[u].y, tt[u].y, Q);
+      R = fmaf(gg[u].x, tt[u].y, R);
+      V = fmaf(gg[u].y, tt[u].x, V);
+    }
+    acc.P += P;
+    acc.Q += Q;
+    acc.R += R;
+    acc.V += V;
+  }
+  const double sg = conj ? -1.0 : 1.0;
+  double re = fma(-sg, acc.Q, acc.P), im = fma(sg, acc.R, acc.V);
+  for (int off = 32; off > 0; off >>= 1) {
+    re += __shfl_xor(re, off);
+    im += __shfl_xor(im, off);
+  }
+  return make_float2((float)re, (float)im);
+}
+
 // The points whose support lies above the plan's max_support but whose window
 // meets no more tiles than the plan allows (they are gridded too): one
-// wavefront per point, the grid read where it lies.  Kept out of the staged
-// region, whose size is the plan's; a plan made for its points has none.
+// wavefront per point.  Kept out of the staged region, whose size is the
+// plan's; a plan made for its points has none.
 __device__ __forceinline__ void win_above(const TiledDev &d, const rcg_pg *__restrict__ pg,
                                           const float2 *__restrict__ grid,
                                           __amdgpu_buffer_rsrc_t rsrc, float2 *__restrict__ vis,
@@ -284,25 +348,9 @@ __device__ __forceinline__ void win_above(const TiledDev &d, const rcg_pg *__res
     point_tiles(r, d.pitch, d.inv_pitch, d.lt, &u0, &v0, &tu0, &tu1, &tv0, &tv1);
     if ((tu1 - tu0 + 1) * (tv1 - tv0 + 1) > d.mpp) continue;
     while (i >= d.pt_off[inst + 1]) inst++;
-    const float2 *g0 = grid + inst * d.gstride + r.cell;
-    const int S = r.supp;
-    float P = 0.f, Q = 0.f, R = 0.f, V = 0.f;
-    for (int q = lane; q < S * S; q += 64) {
-      const int row = q / S, col = q - row * S;
-      const float2 g = g0[(long long)row * d.pitch + col];
-      const float2 t = tap_load(rsrc, (unsigned)(r.tap0 + row * r.stride + col) * 8u, 0);
-      P = fmaf(g.x, t.x, P);
-      Q = fmaf(g.y, t.y, Q);
-      R = fmaf(g.x, t.y, R);
-      V = fmaf(g.y, t.x, V);
-    }
-    const float sg = r.flags & PG_CONJ ? -1.f : 1.f;
-    float re = fmaf(-sg, Q, P), im = fmaf(sg, R, V);
-    for (int off = 32; off > 0; off >>= 1) {
-      re += __shfl_xor(re, off);
-      im += __shfl_xor(im, off);
-    }
-    if (lane == 0) vis[i] = make_float2(re, im);
+    const float2 v = win_point(grid + inst * d.gstride + r.cell, d.pitch, rsrc, r.tap0, r.stride,
+                               r.supp, r.flags & PG_CONJ, lane);
+    if (lane == 0) vis[i] = v;
   }
 }
 
@@ -324,9 +372,26 @@ k_degrid_windows(TiledDev d, int side, int cap, const rcg_pg *__restrict__ pg,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int guess = 0;  // side of the region the last batch needed
   if (threadIdx.x < 2) reg[side * LS + threadIdx.x] = make_float2(0.f, 0.f);
+  // points a record
+  const float share = (float)d.npts / (float)max(d.totals[0], 1);
   for_each_item(d, d.queue + Q_DEGRID, [&](const ItemRange &ir) {
     const int gsz = d.grid_size;
     const float2 *gi = grid + ir.goff;
+    // Of a tile with few points: each by a wavefront (the whole tile alike, so
+    // that a point's sums do not hang on the item its record fell in).
+    if ((float)ir.most * share <= (float)FEW) {
+      for (int k = ir.begin + wave; k < ir.end; k += W) {
+        const int4 rec = uniform_record(d.pairs, k);
+        if (rec.z >= 0) continue;  // not the point's first tile
+        const int S = ((rec.x >> 24) & 63) | ((rec.z >> 24) & 64);
+        const float2 v =
+            win_point(gi + (long long)(ir.tu0 + (rec.x & 63)) * d.pitch + ir.tv0 + ((rec.x >> 6) & 63),
+                      d.pitch, rsrc, rec.y, rec.z & 0xffff, S, (rec.x >> 30) & 1, lane);
+        if (lane == 0) vis[rec.w] = v;
+      }
+      __syncthreads();  // for_each_item's next draw overwrites this one
+      return;
+    }
     // the square of side `to`, without that of side `from`
     auto stage = [&](int from, int to) {
       for (int r = wave; r < to; r += W) {
@@ -439,9 +504,11 @@ const void *win_kernel(int waves)
 
 }  // namespace
 
-bool windows_fit(int T, int max_support)
+bool windows_fit(int T, int max_support, int chunk)
 {
-  return max_support < WIN_BUCKETS && win_lds(T, max_support) <= WIN_LDS;
+  const double tiles = (double)(max_support - 1) / T + 1;
+  return max_support < WIN_BUCKETS && win_lds(T, max_support) <= WIN_LDS &&
+         chunk >= ITEM_POINTS * tiles * tiles;
 }
 
 hipError_t windows_blocks(int T, int max_support, int waves, int *blocks)
