@@ -47,7 +47,7 @@ def parse():
     ap.add_argument("--waves", type=int, default=0,
                     help="wavefronts per gridding workgroup, 1..4 (0: the plan's default)")
     ap.add_argument("--degrid-waves", type=int, default=0,
-                    help="wavefronts per degridding workgroup, 2, 4 or 8 (0: the default 4)")
+                    help="wavefronts per degridding workgroup, 2, 4 or 8 (0: the plan's default)")
     ap.add_argument("--layout", choices=["pairs", "halo", "halo16"], default="pairs",
                     help="record layout of the tiled plan (see rcg_tiled_plan_create_ex)")
     ap.add_argument("--n-times", type=int, default=306)

@@ -737,20 +737,22 @@ k_grid_tiles(TiledDev d, const float2 *__restrict__ vis,
 // at T = 32 a copy is 17 KB, so eight workgroups, all the wavefronts a CU
 // takes, fit one; without the bound below 112 SGPRs left room for seven, and
 // 2038 items of 100 x 100 windows made a second round (1118 against 809 us).
-// Real and imaginary
-// parts lie in planes of their own: 64 lanes on consecutive cells take 9
-// cycles an atomic there and 17 interleaved.  Records come 64 at a time and
-// the next pair's first taps fly while a pair is added; a pair is tested
-// against the table's end once where all of it lies inside.  Measured,
+// Real and imaginary parts lie in planes of their own: 64 lanes on consecutive
+// cells take 9 cycles an atomic there and 17 interleaved.  Records come 64 at
+// a time and the next pair's first taps fly while a pair is added; a pair is
+// tested against the table's end once where all of it lies inside.  Measured,
 // 2,496,960 points of supports 8..48 in chunks of 306 on 2048^2 (330 M taps):
-// 0.65 ms against 0.77 without any of it; 100,000 points of 8 x 8 on 512^2:
-// 0.069 against 0.104 ms.  A private copy per wavefront (two workgroups per CU) took three
-// times as long, the taps of 2-8 slabs loaded together 4-70% more.  A tap
-// index past the table reads nothing and adds nothing.  add: the tile sums are
-// added to the grid's contents (otherwise the grid was zeroed and a tile
-// with a single work item is stored).
+// 0.63 ms against 0.77 without any of it; 100,000 points of 8 x 8 on 512^2:
+// 0.075 against 0.104 ms.  A private copy per wavefront (two workgroups per
+// CU) took three times as long, the taps of 2-8 slabs loaded together 4-70%
+// more.  A tap index past the table reads nothing and adds nothing.  add: the
+// tile sums are added to the grid's contents (otherwise the grid was zeroed
+// and a tile with a single work item is stored).
 
-constexpr int F64_WAVES = 4;  // 2: 3.7 ms, 8: 3.2-3.5 ms on the workload above
+// Gridder / degridder on the two workloads above, ms: 2 wavefronts 0.90 / 1.62
+// and 0.131 / 0.249; 4: 0.63 / 1.35 and 0.075 / 0.147; 8: 0.61 / 1.25 and 0.049
+// / 0.095 (8 was measured on these two alone).
+constexpr int F64_WAVES = 4;
 
 template <int T>
 __global__ void __launch_bounds__(64 * F64_WAVES, T == 64 ? 2 : 8)  // wavefronts per SIMD
@@ -1395,23 +1397,9 @@ rcg_status create_plan(const rcg_geom *geoms, int n_inst, int tile, int chunk, i
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bin_count),
                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   if (e == hipSuccess && !halo) {
-    switch (tile) {
-      case 16:
-        pl->grid_waves = GRID_WAVES;
-        e = tile_kernels<16>(pl->grid_waves, pl->degrid_waves, &pl->grid_blocks,
-                             &pl->degrid_blocks);
-        break;
-      case 32:
-        pl->grid_waves = GRID_WAVES;
-        e = tile_kernels<32>(pl->grid_waves, pl->degrid_waves, &pl->grid_blocks,
-                             &pl->degrid_blocks);
-        break;
-      default:
-        pl->grid_waves = GRID_WAVES;
-        e = tile_kernels<64>(pl->grid_waves, pl->degrid_waves, &pl->grid_blocks,
-                             &pl->degrid_blocks);
-        break;
-    }
+    pl->grid_waves = GRID_WAVES;
+    e = (tile == 16 ? tile_kernels<16> : tile == 32 ? tile_kernels<32> : tile_kernels<64>)(
+        pl->grid_waves, pl->degrid_waves, &pl->grid_blocks, &pl->degrid_blocks);
   }
   pl->windows = !halo && windows_fit(tile, max_support, chunk);
   d.windows = pl->windows ? max_support : 0;

@@ -20,17 +20,18 @@
 // and loads wide.  A window cut at tile edges (k_degrid_tiles) fills 40 of 64
 // lanes with 8 bytes each, and leaves per-tile partial sums to store and add.
 // Measured on the 4096^2 w-projection workload (9,987,840 points, 3.2e9 taps):
-// 1.34 ms, 19 TB/s of taps, against 2.35 + 0.08 ms for k_degrid_tiles and its
-// sums; 16 snapshots of 2048^2 (6.3 M points): 0.89 against 1.65 ms.  With
-// FP32 sums (1.25 ms) 0.85 were the steps (1.15 of 1.35 without loads, so
-// instruction issue and the two workgroups per CU bound it), the rest the sorts
-// and staging of an item.  Variants on the former workload: 16 lanes a point 5%
-// slower, 32 lanes 24% (small windows leave them idle); U = 2 4% slower, 3
-// equal there and 5% slower on the latter; 4 wavefronts per workgroup 36%
-// slower; blocks that all lanes need without the range mask 5% slower; the
-// region staged for the plan's largest support rather than the batch's 12%
-// slower (23% on the latter); supports from the points' pregrid records
-// rather than in the pair records, and staging after the sort, 7% slower.
+// 1.32 ms, 19 TB/s of taps, against 2.35 + 0.08 ms for k_degrid_tiles and its
+// sums; 16 snapshots of 2048^2 (6.3 M points): 0.87 against 1.65 ms.  With
+// FP32 sums (1.26 and 0.82 ms) 0.85 of the former's were the steps, bound by
+// instruction issue and the two workgroups per CU more than by the loads; the
+// rest was the sorts and staging of an item.  Variants on the former workload:
+// 16 lanes a point 5% slower, 32 lanes 24% (small windows leave them idle); U
+// = 2 4% slower, 3 equal there and 5% slower on the latter; 4 wavefronts per
+// workgroup 35% slower (32% on the latter); blocks that all lanes need without
+// the range mask 5% slower; the region staged for the plan's largest support
+// rather than the batch's 12% slower (23% on the latter); supports from the
+// points' pregrid records rather than in the pair records, and staging after
+// the sort, 7% slower.
 #include <algorithm>
 
 #include "rcg_internal.h"
@@ -131,7 +132,7 @@ __device__ __forceinline__ void win_load(Steps &s, Walk &w, int dummy, __amdgpu_
 // chain over the window would be S^2 / 8 long, eight times that of a wavefront
 // per window: relative L2 error of the 4096^2 workload's visibilities, six sets
 // of points, 0.67-2.9e-7 with FP32 sums per call, 0.68-2.2e-7 a wavefront per
-// window, 0.37-1.8e-7 this way, for 1.27 -> 1.34 ms.
+// window, 0.37-1.8e-7 this way, for 1.26 -> 1.32 ms.
 struct Acc {
   double P, Q, R, V;
 };
